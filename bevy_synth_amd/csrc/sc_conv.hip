@@ -5,11 +5,11 @@
 // (crates/burn_flex_gmm/src/wgpu/sparse_conv_kernels.rs K9-K17: one lane per
 // output value re-reading K*Cin inputs and weights from global memory).
 //
-// Every MFMA kernel here computes a tile of 256 query rows x 128 output
-// channels of one group with 4 waves, reduces over (used kernel offset,
-// input-channel chunk) stages, skips offsets no row of the tile uses, and
-// fuses the epilogue (* int8 scale + bias, optional LayerNorm / SiLU over the
-// row, optional residual).  Kernels, by the path that takes them:
+// An MFMA kernel here computes a tile of query rows x output channels of one
+// group (256 x 128 where the call fills the chip with them), reduces over
+// (used kernel offset, input-channel chunk) stages, skips offsets no row of
+// the tile uses, and fuses the epilogue (* int8 scale + bias, optional
+// LayerNorm / SiLU over the row, optional residual).  Kernels, by the path that takes them:
 //   conv_halo_kernel  bf16 activations with a conv plan (sc_plan.hpp) and
 //                     packed weights: the tile's distinct neighbour rows are
 //                     staged in LDS once per 32-channel chunk and every
@@ -19,7 +19,8 @@
 //   conv_v2_kernel    bf16 activations without a plan: neighbour rows
 //                     gathered from global memory per (row, offset), weights
 //                     staged in LDS;
-//   conv_mfma_kernel  f32 activations (v_mfma_f32_32x32x2_f32);
+//   conv_f32_kernel   f32 activations (v_mfma_f32_16x16x4_f32), tiles of 32,
+//                     64 or 128 rows and channels by the size of the call;
 //   conv_scalar_kernel  shapes no tile takes (channel counts that are not
 //                     multiples of the chunk, K > 32, unaligned pointers,
 //                     tensors of 2 GiB or more): one lane per output value.
@@ -212,7 +213,15 @@ static int conv_forward_impl(const sc_conv_config *cfg, int act_dtype, const voi
     // conv kernel.  Otherwise the conv stores its f32 accumulators (into
     // d_out for an f32 output, else into the caller's workspace) and one row
     // kernel applies LayerNorm -> SiLU -> + residual and rounds once.
-    const bool row_fuse = mfma && ln_in_tile(cfg, act_dtype, c2s);
+    // An f32 conv with an f32 output (which needs no workspace) also takes
+    // the row kernel when a tile as wide as the row would leave the chip idle
+    // (the row kernel's 4-15 us against a conv of twice the time or more).
+    bool row_fuse = mfma && ln_in_tile(cfg, act_dtype, c2s);
+    if (row_fuse && act_f32 && out_dtype == SC_DTYPE_F32 && !c2s.skip &&
+        f32_tile(n_q, a.cout_g, groups) < f32_row_tile(a.cout_g)) {
+        const int64_t t = 32 * f32_row_tile(a.cout_g);
+        if ((n_q + t - 1) / t < 224) row_fuse = false;
+    }
     const bool split_ln = want_ln && !row_fuse;
     if (split_ln && c2s.skip)
         return fail(SC_ERR_UNSUPPORTED, "sparse conv: LayerNorm before the parent skip needs the row in one tile");

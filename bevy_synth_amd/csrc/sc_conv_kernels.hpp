@@ -6,12 +6,12 @@
 
 #include "sc_common.hpp"
 #include "sc_plan.hpp"
+#include <algorithm>
 
 namespace sc {
 
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTileRows = 256;  // query rows per workgroup (64 per wave)
@@ -81,6 +81,24 @@ struct ConvArgs {
     int child_plan;
 };
 
+// The f32 tile (conv_f32_kernel): 16-row blocks per wave and side, a workgroup
+// taking 32 kB rows x 32 kB channels.  64 x 64 once those number three
+// quarters of the CUs (188 of them, 6,000 rows x 128 channels: 32 x 32 tiles
+// 66.6 us against 70.8; 256: 292 against 259) and more than 32 channels are
+// computed; 128 x 128 only while one per CU to two are resident at once
+// (30,000 rows x 128, 235 tiles: 237 us against 252 on 64 x 64; 60,000, 469:
+// 429 against 443; 120,000, 938: 853 against 825), and for a channel count
+// that does not leave half the last tile empty.
+inline int f32_tile(int64_t rows, int64_t cols, int groups)
+{
+    auto tiles = [&](int64_t t) { return (rows + t - 1) / t * ((cols + t - 1) / t) * groups; };
+    if (cols <= 32 || tiles(64) <= 192) return 1;
+    const int64_t t4 = tiles(128);
+    return t4 >= 224 && t4 <= 512 && (cols - 1) % 128 >= 64 ? 4 : 2;
+}
+// The smallest tile that holds a whole row of `cols` <= 128 channels.
+inline int f32_row_tile(int64_t cols) { return cols <= 32 ? 1 : (cols <= 64 ? 2 : 4); }
+
 // Header of a packed weight buffer (its first 256 bytes): the shape the
 // weights were packed for.  The planned conv compares it with the call's
 // config before it reads a fragment.
@@ -139,54 +157,7 @@ __device__ inline void widen_i8x16(uint4 q, uint4 &o0, uint4 &o1)
     o1.w = i8pair_to_bf16x2(q.w, 16);
 }
 
-// A fragments of one 32-row block for one stage: NP 16-byte pieces of the
-// gathered row's CB-byte slice.  Piece q of lane half h sits at byte
-// bf16: q*32 + h*16 (one MFMA k-step per piece); f32: h*CB/2 + q*16 (4
-// consecutive k-elements per piece).
-template <int NP>
-struct APiece {
-    uint4 p[NP];
-};
-
-template <bool kF32, int CB>
-__device__ inline int piece_offset(int q, int half)
-{
-    return kF32 ? half * (CB / 2) + q * 16 : q * 32 + half * 16;
-}
-
-
-template <bool kF32, int CB>
-__device__ inline APiece<CB / 32> load_a_pieces(__amdgpu_buffer_rsrc_t r, uint32_t row_off, int kc,
-                                                 int half)
-{
-    APiece<CB / 32> a;
-#pragma unroll
-    for (int q = 0; q < CB / 32; ++q)
-        a.p[q] = bload16(r, row_off + (uint32_t)(kc * CB + piece_offset<kF32, CB>(q, half)));
-    return a;
-}
-
 __device__ inline float u2f(uint32_t u) { return __builtin_bit_cast(float, u); }
-
-// One piece of one 32x32 output block, computed transposed: the weight
-// fragment w (32 output channels) is the MFMA A operand and the gathered
-// input fragment x (32 voxel rows) the B operand, so D[o][r] = sum_k w[o][k]
-// x[r][k] and a lane ends up holding 4 consecutive output channels of one
-// row (packed stores in the epilogue).  bf16 -> one v_mfma_f32_32x32x16_bf16;
-// f32 -> four v_mfma_f32_32x32x2_f32 (element e of each lane half's piece).
-template <bool kF32>
-__device__ inline void mfma_piece(f32x16 &acc, const uint4 &x, const uint4 &w)
-{
-    if constexpr (!kF32) {
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w),
-                                                      __builtin_bit_cast(bf16x8, x), acc, 0, 0, 0);
-    } else {
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(u2f(w.x), u2f(x.x), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(u2f(w.y), u2f(x.y), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(u2f(w.z), u2f(x.z), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(u2f(w.w), u2f(x.w), acc, 0, 0, 0);
-    }
-}
 
 // Packs / unpacks 4 consecutive output values.
 template <typename TO>
@@ -311,354 +282,6 @@ __device__ inline void c2s_store4(const ConvArgs &a, const C2SRow &c, int64_t qr
             if (cc < nv) store_from_f32<TO>(out, base + cc, t[cc]);
     }
 }
-
-// ------------------------------------------------------------- MFMA tile
-
-// Per-tile list of kernel offsets (K <= 32) used by at least one row of the
-// tile: per-thread bit masks OR-reduced across the wave, one LDS atomic per
-// wave, then a serial compaction by thread 0.
-__device__ inline int build_offset_list(const int32_t *map_tile, int nrows, int K, int64_t n_in,
-                                        uint32_t *s_kmask, int16_t *s_klist, int *s_nk)
-{
-    const int tid = threadIdx.x, lane = tid & 63;
-    for (int i = tid; i < (K + 31) / 32; i += blockDim.x) s_kmask[i] = 0;
-    __syncthreads();
-    {
-        // The tile's map block is contiguous: read it as int4, four loads in
-        // flight per thread before any is inspected.
-        uint32_t m = 0;
-        const int total = nrows * K;
-        const int4 *m4 = reinterpret_cast<const int4 *>(map_tile);
-        const int n4 = total >> 2;
-        for (int base = tid; base < n4; base += 4 * (int)blockDim.x) {
-            int4 v[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int i4 = base + u * (int)blockDim.x;
-                v[u] = i4 < n4 ? m4[i4] : make_int4(-1, -1, -1, -1);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int e = 4 * (base + u * (int)blockDim.x);
-                const int32_t vv[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    if (vv[c] >= 0 && vv[c] < n_in) m |= 1u << ((e + c) % K);
-            }
-        }
-        for (int e = 4 * n4 + tid; e < total; e += blockDim.x) {
-            const int32_t v = map_tile[e];
-            if (v >= 0 && v < n_in) m |= 1u << (e % K);
-        }
-        uint32_t lo = (uint32_t)m;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) lo |= __shfl_xor(lo, off, 64);
-        if (lane == 0 && lo) atomicOr(&s_kmask[0], lo);
-    }
-    __syncthreads();
-    if (tid == 0) {
-        int nk = 0;
-        for (int k = 0; k < K; ++k)
-            if (s_kmask[k >> 5] & (1u << (k & 31))) s_klist[nk++] = (int16_t)k;
-        *s_nk = nk;
-    }
-    __syncthreads();
-    return *s_nk;
-}
-
-
-// LDS table of the byte offsets (in the input) of the neighbour rows of the
-// tile: s_aoff[ki][r] for used offset ki and tile row r (thread r fills row r);
-// kOobOffset for an absent neighbour or a row past the end.
-__device__ inline void fill_row_offsets(const int32_t *map_tile, int nrows, int K, int64_t n_in,
-                                        uint32_t row_bytes, const int16_t *s_klist, int nk,
-                                        uint32_t (*s_aoff)[kTileRows])
-{
-    const int r = threadIdx.x;  // kThreads == kTileRows
-    const int32_t *mrow = map_tile + (int64_t)min(r, nrows - 1) * K;
-    for (int k0 = 0; k0 < nk; k0 += 8) {
-        int32_t v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = k0 + u < nk ? mrow[s_klist[k0 + u]] : -1;
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (k0 + u < nk)
-                s_aoff[k0 + u][r] =
-                    (r < nrows && v[u] >= 0 && v[u] < n_in) ? (uint32_t)v[u] * row_bytes : kOobOffset;
-    }
-    __syncthreads();
-}
-
-// Tile = 256 query rows x 128 output channels of one group; 4 waves, wave w
-// owns rows [64w, 64w+64) x all 128 channels (2 x 4 MFMA 32x32 blocks, 128
-// f32 accumulators per lane).  CB = bytes of a row's reduction slice per
-// stage (64 or 128); a stage is (used offset ki, input chunk kc).
-//
-// Prologue: the offsets used by the tile, then an LDS table of the byte
-// offsets of every (used offset, row) neighbour row in the input (an
-// out-of-range offset for absent neighbours), so the main loop issues no map
-// loads.  Main loop: a two-half software pipeline with no branches -- each
-// half issues the next stage's weight loads (-> LDS after the MFMAs) and A
-// loads (-> the other register set), then runs this stage's MFMAs.  The
-// stage count is padded to even with a zero-weight stage.
-template <typename TA, typename TW, typename TO, int CB>
-__global__ __launch_bounds__(kThreads, 2) void conv_mfma_kernel(ConvArgs args)
-{
-    constexpr bool kF32 = sizeof(TA) == 4;
-    constexpr int kBK = CB / (int)sizeof(TA);  // reduction elements per stage
-    constexpr bool kI8 = sizeof(TW) == 1;
-    constexpr int kRows = kTileRows;
-    constexpr int NP = CB / 32;                 // A/B pieces per lane per row block
-    constexpr int kStride = CB + 16;            // LDS pitch of one output channel
-    constexpr int kWBytes = kBK * (int)sizeof(TW);  // weight bytes per channel per stage
-    constexpr int kWPieces = kWBytes / 16;      // 16-byte weight pieces per channel
-    constexpr int kBPerThread = kBN * kWPieces / kThreads;
-    static_assert(kBPerThread >= 1, "weight pieces per thread");
-
-    __shared__ __attribute__((aligned(16))) unsigned char s_b[2][kBN * kStride];
-    __shared__ uint32_t s_aoff[kMaxTableK][kRows];
-    __shared__ uint32_t s_kmask[kMaxTableK / 32 + 1];
-    __shared__ int16_t s_klist[kMaxTableK];
-    __shared__ int s_nk;
-
-    const TA *input = static_cast<const TA *>(args.input);
-    const TW *weight = static_cast<const TW *>(args.weight);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6, half = lane >> 5;
-    const int K = args.K;
-
-    const int tile = tile_for_block(blockIdx.x, gridDim.x);
-    const int64_t row0 = (int64_t)tile * kRows;
-    const int o0 = blockIdx.y * kBN;  // within the group
-    const int g = blockIdx.z;
-    const int64_t in_col0 = (int64_t)g * args.cin_g;
-    const int64_t out_col0 = (int64_t)g * args.cout_g;
-    const int nrows = (int)min<int64_t>(kRows, args.n_q - row0);
-    const int32_t *map_tile = args.map ? args.map + row0 * K : nullptr;
-    const int64_t n_in = args.n_in;
-    const uint32_t row_bytes = (uint32_t)(args.cin * (int64_t)sizeof(TA));
-
-    int nk;
-    if (args.map) {
-        nk = build_offset_list(map_tile, nrows, K, n_in, s_kmask, s_klist, &s_nk);
-        fill_row_offsets(map_tile, nrows, K, n_in, row_bytes, s_klist, nk, s_aoff);
-    } else {
-        // no map: the dense linear (K = 1), query row r reads input row r
-        nk = 1;
-        if (tid == 0) s_klist[0] = 0;
-        s_aoff[0][tid] = tid < nrows && row0 + tid < n_in ? (uint32_t)(row0 + tid) * row_bytes : kOobOffset;
-        __syncthreads();
-    }
-
-    const int nkc = args.cin_g / kBK;  // chunks per offset
-    const int S = nk * nkc;
-    const int S2 = S + (S & 1);
-
-    f32x16 acc[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-    if (S > 0) {
-        const int ar0 = wave * 64 + (lane & 31), ar1 = ar0 + 32;
-        const __amdgpu_buffer_rsrc_t a_rsrc =
-            make_rsrc(input + in_col0, (uint32_t)(n_in * row_bytes - in_col0 * (int64_t)sizeof(TA)));
-        const __amdgpu_buffer_rsrc_t w_rsrc =
-            make_rsrc(weight, (uint32_t)(args.cout * (int64_t)K * args.cin_g * (int64_t)sizeof(TW)));
-
-        // Weight pieces: index t + 256*i -> channel idx / kWPieces, piece idx % kWPieces.
-        uint32_t w_base[kBPerThread];
-#pragma unroll
-        for (int i = 0; i < kBPerThread; ++i) {
-            const int idx = tid + kThreads * i;
-            const int ch = idx / kWPieces, pc = idx % kWPieces;
-            w_base[i] = o0 + ch < args.cout_g
-                            ? (uint32_t)((out_col0 + o0 + ch) * (int64_t)K * args.cin_g * (int64_t)sizeof(TW)) + pc * 16
-                            : kOobOffset;
-        }
-        const uint32_t w_k_bytes = (uint32_t)(args.cin_g * (int64_t)sizeof(TW));
-        uint4 rb[kBPerThread];
-        // Loads of stage t (t >= S: zero weights, zero A).
-        auto load_stage = [&](int t, APiece<NP> &f0, APiece<NP> &f1) {
-            const bool live = t < S;
-            const int tt = live ? t : 0;
-            const int ki = tt / nkc, kc = tt - ki * nkc;
-            const int k = s_klist[ki];
-            const uint32_t wk = (uint32_t)k * w_k_bytes + (uint32_t)(kc * kWBytes);
-#pragma unroll
-            for (int i = 0; i < kBPerThread; ++i) rb[i] = bload16(w_rsrc, live ? w_base[i] + wk : kOobOffset);
-            const uint32_t o_a0 = live ? s_aoff[ki][ar0] : kOobOffset;
-            const uint32_t o_a1 = live ? s_aoff[ki][ar1] : kOobOffset;
-            f0 = load_a_pieces<kF32, CB>(a_rsrc, o_a0, kc, half);
-            f1 = load_a_pieces<kF32, CB>(a_rsrc, o_a1, kc, half);
-        };
-        auto store_b = [&](int buf) {
-            unsigned char *b = s_b[buf];
-#pragma unroll
-            for (int i = 0; i < kBPerThread; ++i) {
-                const int idx = tid + kThreads * i;
-                const int ch = idx / kWPieces, pc = idx % kWPieces;
-                if constexpr (kI8) {
-                    uint4 w0, w1;
-                    widen_i8x16(rb[i], w0, w1);
-                    *reinterpret_cast<uint4 *>(b + ch * kStride + pc * 32) = w0;
-                    *reinterpret_cast<uint4 *>(b + ch * kStride + pc * 32 + 16) = w1;
-                } else {
-                    *reinterpret_cast<uint4 *>(b + ch * kStride + pc * 16) = rb[i];
-                }
-            }
-        };
-        const int bcol = lane & 31;
-        auto compute = [&](int buf, const APiece<NP> &c0, const APiece<NP> &c1) {
-            const unsigned char *b = s_b[buf];
-#pragma unroll
-            for (int q = 0; q < NP; ++q) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint4 bq = *reinterpret_cast<const uint4 *>(
-                        b + (j * 32 + bcol) * kStride + piece_offset<kF32, CB>(q, half));
-                    mfma_piece<kF32>(acc[0][j], c0.p[q], bq);
-                    mfma_piece<kF32>(acc[1][j], c1.p[q], bq);
-                }
-            }
-        };
-
-        APiece<NP> x0, x1, y0, y1;
-        load_stage(0, x0, x1);
-        store_b(0);
-        __syncthreads();
-        // sched_barrier keeps the next stage's loads ahead of this stage's
-        // MFMAs (the scheduler would otherwise sink them below).
-        for (int t = 0; t < S2; t += 2) {
-            load_stage(t + 1, y0, y1);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(0, x0, x1);
-            store_b(1);
-            __syncthreads();
-            load_stage(t + 2, x0, x1);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(1, y0, y1);
-            store_b(0);
-            __syncthreads();
-        }
-    }
-
-    // ---- epilogue.  32x32 MFMA result layout (transposed product): lane l,
-    //      element e -> output channel 8*(e/4) + 4*(l/32) + e%4 of the block,
-    //      voxel row l%32.  Each run of 4 elements is 4 consecutive channels;
-    //      lanes l and l^32 together hold all channels of a row.
-    TO *__restrict__ out = static_cast<TO *>(args.out);
-    const TO *__restrict__ res = static_cast<const TO *>(args.residual);
-    const bool vec_ok = args.vec_out != 0;
-    // bias / int8 scale per channel, applied to both row blocks at once
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int o = o0 + j * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
-            const bool ok = o < args.cout_g;
-            const float bias = (args.bias && ok) ? args.bias[out_col0 + o] : 0.f;
-            const float scale = (kI8 && args.w_scale && ok) ? args.w_scale[out_col0 + o] : 1.f;
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                acc[i][j][e] = ok ? (kI8 ? acc[i][j][e] * scale + bias : acc[i][j][e] + bias) : 0.f;
-        }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int r = wave * 64 + i * 32 + (lane & 31);
-        if (r >= nrows) continue;  // lanes l and l^32 share r: both skip together
-        const int64_t rowbase = (row0 + r) * args.cout + out_col0;
-        if (args.ln) {
-            // Two-pass f32 statistics over the row's Cout channels (the
-            // reference's layer_norm_row_stats, wgpu/ops.rs:162-187).
-            float s = 0.f;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) s += acc[i][j][e];
-            s += __shfl_xor(s, 32, 64);
-            const float inv_c = 1.0f / (float)args.cout_g;
-            const float mean = s * inv_c;
-            float q = 0.f;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int o = o0 + j * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
-                    const float d = acc[i][j][e] - mean;
-                    q += o < args.cout_g ? d * d : 0.f;
-                }
-            q += __shfl_xor(q, 32, 64);
-            const float inv_std = rsqrt_f32(q * inv_c + args.ln_eps);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int o = o0 + j * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
-                    const bool ok = o < args.cout_g;
-                    float t = (acc[i][j][e] - mean) * inv_std;
-                    if (args.ln_w && ok) t *= args.ln_w[o];
-                    if (args.ln_b && ok) t += args.ln_b[o];
-                    acc[i][j][e] = t;
-                }
-        }
-        if (args.silu) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const float t = acc[i][j][e];
-                    acc[i][j][e] = silu_f32(t);
-                }
-        }
-        if (args.scatter_rows || args.skip_idx) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int e4 = 0; e4 < 4; ++e4) {
-                    const int oc = o0 + j * 32 + 8 * e4 + 4 * half;
-                    if (oc >= args.cout_g) continue;
-                    float v[4];
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) v[c] = acc[i][j][4 * e4 + c];
-                    c2s_store4<TO>(args, c2s_row<TO>(args, row0 + r), row0 + r, (int)(out_col0 + oc),
-                                   min(4, args.cout_g - oc), v, vec_ok);
-                }
-            continue;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                const int oc = o0 + j * 32 + 8 * e4 + 4 * half;  // first of 4 channels
-                float v[4];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) v[c] = acc[i][j][4 * e4 + c];
-                if (vec_ok && oc + 3 < args.cout_g) {
-                    typename Out4<TO>::V *dst = reinterpret_cast<typename Out4<TO>::V *>(out + rowbase + oc);
-                    if (res) {
-                        float rv[4];
-                        Out4<TO>::unpack(*reinterpret_cast<const typename Out4<TO>::V *>(res + rowbase + oc), rv);
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) v[c] += rv[c];
-                    }
-                    *dst = Out4<TO>::pack(v);
-                } else {
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        if (oc + c >= args.cout_g) continue;
-                        float t = v[c];
-                        if (res) t += load_as_f32<TO>(res, rowbase + oc + c);
-                        store_from_f32<TO>(out, rowbase + oc + c, t);
-                    }
-                }
-            }
-    }
-}
-
 
 // ------------------------------------------------------ bf16 tile, v2
 //
@@ -2170,6 +1793,8 @@ __global__ __launch_bounds__(256) void conv_scalar_kernel(ConvArgs args)
     }
 }
 
+#include "sc_conv_f32.hpp"
+
 // 16-bit activations through the v2 tile: 128-byte stages when the group's
 // input channels allow it, else 64-byte stages with a deeper A prefetch.
 // int8 weights always take the 64-byte stages: their register staging of the
@@ -2191,7 +1816,6 @@ template <typename TA, typename TW, typename TO>
 int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipStream_t s)
 {
     if (mfma) {
-        const bool wide = a.cin_g % (128 / (int)sizeof(TA)) == 0;
         const int64_t tiles = (a.n_q + kTileRows - 1) / kTileRows;
         const int64_t ntile = (a.cout_g + kBN - 1) / kBN;
         if (tiles > INT32_MAX || ntile > 65535 || groups > 65535)
@@ -2300,12 +1924,9 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                 launch_v2<TA, TW, TO>(a, grid, s);
             }
         } else {
-            if (wide)
-                conv_mfma_kernel<TA, TW, TO, 128><<<grid, kThreads, 0, s>>>(a);
-            else
-                conv_mfma_kernel<TA, TW, TO, 64><<<grid, kThreads, 0, s>>>(a);
+            return launch_f32<TO>(a, groups, s);
         }
-        SC_LAUNCH_CHECK("conv_mfma_kernel launch");
+        SC_LAUNCH_CHECK("conv_v2_kernel launch");
     } else {
         conv_scalar_kernel<TA, TW, TO><<<grid_for(a.n_q * a.cout, 256, 65536), 256, 0, s>>>(a);
         SC_LAUNCH_CHECK("conv_scalar_kernel launch");

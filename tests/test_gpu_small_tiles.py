@@ -1,0 +1,110 @@
+"""GPU tests of the conv tiles that calls below a full chip take, at the edges
+of their tiles and of the rules that choose them, against the fp64 definition
+on the same rounded operands:
+
+* conv_f32_kernel: tiles of 32, 64 or 128 rows and channels.
+
+bf16 / f16 outputs are held to half an ulp of the output plus the f32 bound;
+f32 outputs to 2e-5: the sum of 27 * Cin products in f32, whose error in any
+order is below (27 * Cin) * 2^-24 of the sum of magnitudes and in practice near
+its square root (about 2e-6 here)."""
+import numpy as np
+import pytest
+import torch
+
+from bevy_synth_amd import flex_gmm as F
+from bevy_synth_amd import synth
+from tests.test_gpu_plan import bf16_dev, dev, ocfg, rbf
+from tests.tolerance import assert_close
+
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.float32: 2e-5, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11 + 2e-5}
+
+
+def shell(n, seed=0):
+    """n rows of a thick shell in (b, x, y, z) order."""
+    r = 6.0
+    while True:
+        c = synth.sphere_shell_coords(int(2 * r) + 8, r, 1.5, (r + 4,) * 3)
+        if len(c) >= n:
+            return np.ascontiguousarray(c[:n])
+        r *= 1.3
+
+
+def conv_case(oracle, n, cin, cout, dtype, w="same", planned=False, ln=False, residual=False, groups=1, out=None,
+              kernel=(3, 3, 3), coords=None, n_q=None, rows=None):
+    rng = np.random.default_rng((n or 0) + 7 * cin + cout)
+    cfg = F.SparseSubmConvConfig(cin, cout, *kernel, groups=groups)
+    coords = shell(n) if coords is None else coords
+    n = len(coords)
+    K = F.kernel_rows(cfg)
+    f16 = dtype == torch.float16
+    rnd = (lambda a: a) if dtype == torch.float32 else (oracle.f16_round if f16 else rbf)
+    to = dev if dtype == torch.float32 else ((lambda a: dev(a).half()) if f16 else bf16_dev)
+    x = rnd(synth.normal_f32(rng, (n, cin)))
+    cg = cin // groups
+    if w == "i8":
+        q, scale = synth.int8_weight(rng, cout, K, cg)
+        scale = (scale / np.sqrt(K * cg / 3)).astype(np.float32)
+        wv, wd, sd = q.astype(np.float64) * scale[:, None, None], dev(q), dev(scale)
+    else:
+        wv = rnd(synth.conv_weight(rng, cout, K, cg, 1 / np.sqrt(K * cg)))
+        wd, sd = to(wv), None
+    b = synth.normal_f32(rng, cout, 0.1)
+    nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, dev(coords), query_rows=n_q)
+    n_q = n if n_q is None else n_q
+    od = dtype if out is None else out
+    res = rbf(synth.normal_f32(rng, (n_q, cout))) if residual else None  # exact in bf16 and f32
+    res = oracle.f16_round(res) if residual and f16 else res
+    plan = F.build_conv_plan(cfg, dev(coords), nbr) if planned else None
+    packed = F.pack_conv_weight(cfg, wd) if planned else None
+    got = F.sparse_subm_conv_forward(cfg, to(x), nbr, wd, dev(b), sd, out_dtype=od,
+                                     residual=None if res is None else dev(res).to(od), layer_norm=ln, silu=ln,
+                                     plan=plan, packed_weight=packed).float().cpu().numpy()
+    if planned:
+        F.conv_plan_check(plan)
+    m = nbr.cpu().numpy()
+    sel = np.arange(n_q) if rows is None else rows(n_q)
+    exp = oracle.conv_gemm_f64(ocfg(oracle, cfg), np.asarray(wv, np.float32), b, x, m[sel]) if w != "i8" else \
+        oracle.conv_gemm_f64(ocfg(oracle, cfg), q, b, x, m[sel], w_scale=scale)
+    if ln:
+        exp = exp - exp.mean(1, keepdims=True)
+        exp = exp / np.sqrt((exp * exp).mean(1, keepdims=True) + 1e-6)
+        exp = exp / (1 + np.exp(-exp))
+    if res is not None:
+        exp = exp + res[sel]
+    assert_close(got[sel], exp, TOL[od] if not ln else max(TOL[od], 4e-5), f"{n} rows {cin}->{cout}")
+
+
+@pytest.mark.parametrize("n,cin,cout,groups,ln,kernel,out", [
+    (1, 16, 64, 1, False, (3, 3, 3), None),
+    (31, 16, 24, 1, True, (3, 3, 3), None),
+    (33, 48, 33, 1, False, (3, 3, 3), None),      # an odd slice count in the two-slice stages
+    (6144, 32, 128, 1, True, (3, 3, 3), None),    # 192 tiles of 64 x 64: the last on 32 x 32
+    (6145, 32, 128, 1, True, (3, 3, 3), None),    # and the first past it
+    (12289, 16, 65, 1, False, (3, 1, 1), None),
+    (28672, 16, 128, 1, True, (3, 3, 1), None),   # 224 tiles of 128 x 128
+    (28545, 16, 100, 1, False, (3, 3, 1), None),
+    (3000, 32, 128, 1, True, (3, 3, 3), torch.bfloat16),  # LayerNorm stays in the tile: no workspace
+    (900, 64, 96, 2, False, (3, 3, 3), None),
+    (500, 64, 129, 1, False, (1, 1, 1), None),
+    (40, 16, 40, 1, False, (2, 4, 4), None),      # 32 offsets
+])
+def test_f32_tile_edges(oracle, n, cin, cout, groups, ln, kernel, out):
+    conv_case(oracle, n, cin, cout, torch.float32, ln=ln, residual=True, groups=groups, kernel=kernel, out=out,
+              rows=lambda q: np.unique(np.r_[0:min(q, 400), max(0, q - 400):q]))
+
+
+def test_f32_tile_isolated_rows(oracle):
+    """Rows without any neighbour but one offset, and a map of -1 only."""
+    cfg = F.SparseSubmConvConfig(16, 48)
+    rng = np.random.default_rng(3)
+    x, w, b = synth.normal_f32(rng, (70, 16)), synth.conv_weight(rng, 48, 27, 16, 0.1), synth.normal_f32(rng, 48)
+    nbr = np.full((70, 27), -1, np.int32)
+    got = F.sparse_subm_conv_forward(cfg, dev(x), dev(nbr), dev(w), dev(b)).cpu().numpy()
+    assert np.array_equal(got, np.broadcast_to(b, got.shape))
+    nbr[69, 26] = 3
+    got = F.sparse_subm_conv_forward(cfg, dev(x), dev(nbr), dev(w), dev(b)).cpu().numpy()
+    assert_close(got, oracle.conv_gemm_f64(ocfg(oracle, cfg), w, b, x, nbr), TOL[torch.float32])
+
