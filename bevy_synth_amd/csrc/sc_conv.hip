@@ -19,6 +19,9 @@
 //   conv_v2_kernel    bf16 activations without a plan: neighbour rows
 //                     gathered from global memory per (row, offset), weights
 //                     staged in LDS;
+//   conv_rows_kernel  16-bit activations, calls too small to fill the chip
+//                     with 256-row tiles: operands straight from global
+//                     memory, up to four waves sharing a block's reduction;
 //   conv_f32_kernel   f32 activations (v_mfma_f32_16x16x4_f32), tiles of 32,
 //                     64 or 128 rows and channels by the size of the call;
 //   conv_scalar_kernel  shapes no tile takes (channel counts that are not

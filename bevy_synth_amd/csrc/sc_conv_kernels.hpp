@@ -7,6 +7,7 @@
 #include "sc_common.hpp"
 #include "sc_plan.hpp"
 #include <algorithm>
+#include <type_traits>
 
 namespace sc {
 
@@ -1793,6 +1794,7 @@ __global__ __launch_bounds__(256) void conv_scalar_kernel(ConvArgs args)
     }
 }
 
+#include "sc_conv_rows.hpp"
 #include "sc_conv_f32.hpp"
 
 // 16-bit activations through the v2 tile: 128-byte stages when the group's
@@ -1822,6 +1824,9 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
             return fail(SC_ERR_OVERFLOW, "sparse conv grid overflow");
         dim3 grid((unsigned)tiles, (unsigned)ntile, (unsigned)groups);
         if constexpr (sizeof(TA) == 2) {
+            ConvArgs r = a;  // the row-block tile's arguments
+            if (sizeof(TW) != 1) r.w_scale = nullptr;
+            if (!(plan && a.wpack)) r.wpack = nullptr;
             if (plan && a.wpack) {
                 // Halo-staged tiles (a tile whose halo overflowed gathers
                 // its operands from global memory in the same launch).
@@ -1847,6 +1852,19 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                 h.plan_hdr = pv.hdr;
                 h.tile_child = pv.tile_child;
                 if (sizeof(TW) != 1) h.w_scale = nullptr;
+                // a child plan is sized by a bound on the children, of which
+                // about half are active
+                const int64_t rows = a.child_plan ? n_tiles * kPlanTileRows : a.n_q;
+                if (const RowsCut cut = rows_cut(a.child_plan ? a.scatter_n / 2 : rows, cols, groups); cut.kI) {
+                    r.plan_hdr = pv.hdr;
+                    if (a.child_plan) {
+                        r.tile_child = pv.tile_child;
+                        r.perm = pv.order;
+                    }
+                    // packed int8 weights are bf16
+                    using TP = std::conditional_t<sizeof(TW) == 1, uint16_t, TW>;
+                    return launch_rows<TA, TP, TO>(r, cut, rows, cols, groups, s);
+                }
                 if (cols <= 64) {  // 64-channel tiles: no half-empty MFMA tile
                     hgrid.y = (unsigned)((cols + 63) / 64);
                     if (a.ln)
@@ -1871,6 +1889,9 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                 const bool wide_tile = a.cout_g > 128 && a.cout_g <= 256 && !a.ln;
                 const int64_t ncol = (a.cout_g + (wide_tile ? 255 : 127)) / (wide_tile ? 256 : 128);
                 if (tiles * ncol > INT32_MAX) return fail(SC_ERR_OVERFLOW, "dense linear grid overflow");
+                if (!a.child_plan)
+                    if (const RowsCut cut = rows_cut(a.n_q, a.cout_g, 1); cut.kI)
+                        return launch_rows<TA, TW, TO>(r, cut, a.n_q, a.cout_g, 1, s);
                 const dim3 dgrid((unsigned)(tiles * ncol), 1, 1);
                 // row-contiguous stores through LDS: 16-bit output, 8-channel
                 // pieces aligned in the output rows, residual aligned
@@ -1886,6 +1907,12 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                     h.plan_hdr = pv.hdr;
                     h.perm = pv.order;
                     h.tile_child = pv.tile_child;
+                    if (const RowsCut cut = rows_cut(a.scatter_n, a.child_ch, 1); cut.kI) {
+                        r.plan_hdr = pv.hdr;
+                        r.perm = pv.order;
+                        r.tile_child = pv.tile_child;
+                        return launch_rows<TA, TW, TO>(r, cut, CL.n_main * kPlanTileRows, a.child_ch, 1, s);
+                    }
                     const int64_t lgrid = CL.n_main * (a.child_ch / 128);
                     if (lgrid > INT32_MAX) return fail(SC_ERR_OVERFLOW, "dense linear grid overflow");
                     const dim3 lg((unsigned)lgrid, 1, 1);
@@ -1921,6 +1948,8 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                 }
                 SC_LAUNCH_CHECK("dense_gemm_kernel launch");
             } else {
+                if (const RowsCut cut = rows_cut(a.n_q, a.cout_g, groups); cut.kI)
+                    return launch_rows<TA, TW, TO>(r, cut, a.n_q, a.cout_g, groups, s);
                 launch_v2<TA, TW, TO>(a, grid, s);
             }
         } else {

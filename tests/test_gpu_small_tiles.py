@@ -2,7 +2,10 @@
 of their tiles and of the rules that choose them, against the fp64 definition
 on the same rounded operands:
 
-* conv_f32_kernel: tiles of 32, 64 or 128 rows and channels.
+* conv_rows_kernel (16-bit activations): 1, 2 or 4 row blocks per wave, by the
+  number of 16-row x 64-channel blocks (256, 512, 2,048);
+* conv_f32_kernel: tiles of 32, 64 or 128 rows and channels;
+* the halo-staged tiles at channel counts that keep few rows on them.
 
 bf16 / f16 outputs are held to half an ulp of the output plus the f32 bound;
 f32 outputs to 2e-5: the sum of 27 * Cin products in f32, whose error in any
@@ -14,7 +17,7 @@ import torch
 
 from bevy_synth_amd import flex_gmm as F
 from bevy_synth_amd import synth
-from tests.test_gpu_plan import bf16_dev, dev, ocfg, rbf
+from tests.test_gpu_plan import bf16_dev, cluster_coords, dev, ocfg, rbf
 from tests.tolerance import assert_close
 
 pytestmark = pytest.mark.gpu
@@ -77,6 +80,30 @@ def conv_case(oracle, n, cin, cout, dtype, w="same", planned=False, ln=False, re
     assert_close(got[sel], exp, TOL[od] if not ln else max(TOL[od], 4e-5), f"{n} rows {cin}->{cout}")
 
 
+# rows at and past the ends of 16-, 32- and 64-row tiles, and on both sides of
+# the rule's block counts (64 output channels: one block per 16 rows)
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 65, 4096, 4097, 8192, 8193, 32768, 32769])
+@pytest.mark.parametrize("planned", [False, True])
+def test_rows_tile_edges(oracle, n, planned):
+    conv_case(oracle, n, 32, 64, torch.bfloat16, planned=planned, residual=n % 2 == 1,
+              rows=lambda q: np.unique(np.r_[0:min(q, 300), max(0, q - 300):q]))
+
+
+@pytest.mark.parametrize("dtype,w,cin,cout,groups,ln,out,n,planned", [
+    (torch.float16, "same", 64, 96, 1, True, None, 1000, True),     # LayerNorm over two 64-channel columns
+    (torch.bfloat16, "same", 64, 128, 1, True, None, 5000, False),
+    (torch.bfloat16, "same", 32, 100, 1, True, torch.float32, 9001, True),
+    (torch.bfloat16, "i8", 96, 24, 1, False, None, 700, False),     # int8 weights widened in registers
+    (torch.bfloat16, "i8", 64, 72, 1, False, torch.float32, 700, True),
+    (torch.float16, "same", 64, 7, 1, False, torch.float32, 333, False),  # scalar stores
+    (torch.bfloat16, "same", 128, 192, 2, False, None, 777, True),  # groups
+    (torch.bfloat16, "same", 128, 192, 2, False, None, 777, False),
+    (torch.bfloat16, "same", 512, 256, 1, False, None, 3000, True),
+])
+def test_rows_tile_forms(oracle, dtype, w, cin, cout, groups, ln, out, n, planned):
+    conv_case(oracle, n, cin, cout, dtype, w, planned, ln, not ln, groups, out)
+
+
 @pytest.mark.parametrize("n,cin,cout,groups,ln,kernel,out", [
     (1, 16, 64, 1, False, (3, 3, 3), None),
     (31, 16, 24, 1, True, (3, 3, 3), None),
@@ -108,3 +135,15 @@ def test_f32_tile_isolated_rows(oracle):
     got = F.sparse_subm_conv_forward(cfg, dev(x), dev(nbr), dev(w), dev(b)).cpu().numpy()
     assert_close(got, oracle.conv_gemm_f64(ocfg(oracle, cfg), w, b, x, nbr), TOL[torch.float32])
 
+
+@pytest.mark.parametrize("cout,form", [(1024, "plain"), (640, "residual")])
+def test_halo_tiles_few_rows(oracle, cout, form):
+    """Enough output channels that few rows stay on the halo-staged tiles:
+    tiles over the LDS budget, mixed with others, and a partial last tile."""
+    coords = cluster_coords(1300)
+    extra = shell(4100).copy()
+    extra[:, 1] += 200
+    centres, rest = coords[:1300], coords[1300:]
+    both = np.concatenate([centres, extra, rest])
+    conv_case(oracle, None, 32, cout, torch.bfloat16, planned=True, residual=form == "residual", coords=both,
+              n_q=1300 + len(extra), rows=lambda q: np.unique(np.r_[0:300, 1200:1500, q - 300:q]))
