@@ -5,6 +5,8 @@ on the same rounded operands:
 * conv_rows_kernel (16-bit activations): 1, 2 or 4 row blocks per wave, by the
   number of 16-row x 64-channel blocks (256, 512, 2,048);
 * conv_f32_kernel: tiles of 32, 64 or 128 rows and channels;
+* linear_skinny_rows_kernel: rows around a wave's 64, channels around its 128
+  bytes;
 * the halo-staged tiles at channel counts that keep few rows on them.
 
 bf16 / f16 outputs are held to half an ulp of the output plus the f32 bound;
@@ -134,6 +136,17 @@ def test_f32_tile_isolated_rows(oracle):
     nbr[69, 26] = 3
     got = F.sparse_subm_conv_forward(cfg, dev(x), dev(nbr), dev(w), dev(b)).cpu().numpy()
     assert_close(got, oracle.conv_gemm_f64(ocfg(oracle, cfg), w, b, x, nbr), TOL[torch.float32])
+
+
+@pytest.mark.parametrize("rows,cin,cout,dtype", [
+    (1, 8, 8, torch.float16), (63, 64, 1, torch.bfloat16), (64, 72, 8, torch.bfloat16), (65, 4, 8, torch.float32),
+    (129, 36, 5, torch.float32), (1000, 136, 7, torch.float16)])
+def test_skinny_rows_edges(rows, cin, cout, dtype):
+    rng = np.random.default_rng(rows + cin)
+    x = dev(synth.normal_f32(rng, (rows, cin))).to(dtype)
+    w, b = synth.normal_f32(rng, (cout, cin)), synth.normal_f32(rng, cout)
+    got = F.linear_skinny(x, dev(w), dev(b)).cpu().numpy()
+    assert_close(got, x.double().cpu().numpy() @ w.T.astype(np.float64) + b, TOL[torch.float32])
 
 
 @pytest.mark.parametrize("cout,form", [(1024, "plain"), (640, "residual")])
