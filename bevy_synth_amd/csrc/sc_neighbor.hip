@@ -942,6 +942,152 @@ __global__ __launch_bounds__(256) void nm_query_kernel(const int4 *__restrict__ 
     }
 }
 
+// The whole build in one launch, for coord sets that fit a workgroup's LDS
+// and at most 32 offsets: every workgroup loads all the coords, hashes them
+// into its own LDS table of row numbers (slots compared through the coords,
+// the lowest row of duplicates kept), and maps its own kSmallQuery rows; the
+// first also derives the header the four-kernel build writes (bbox, order
+// bits, table mode).  A set of a few hundred rows is bound by launches: 607
+// sorted rows took the four kernels 16.3 us, this one 8.6; 4,096 rows 17.7
+// and 12.9; 607 and 4,096 rows of a box beyond the dense grid 43.7 and 8.5,
+// 53.5 and 14.2.  More rows than that do not fit (coords 64 KB, 4 slots a
+// row 64 KB; 2 slots a row at 4,096 rows took 21 us).
+constexpr int kSmallRows = 4096;
+constexpr int kSmallSlots = 4 * kSmallRows;
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallQuery = 64;
+constexpr int kSmallMaxK = 32;
+
+__device__ inline uint32_t small_hash(int32_t b, int32_t x, int32_t y, int32_t z)
+{
+    uint32_t v = (uint32_t)x * 0x9E3779B1u + (uint32_t)y * 0x85EBCA6Bu + (uint32_t)z * 0xC2B2AE35u +
+                 (uint32_t)b * 0x27D4EB2Fu;
+    v ^= v >> 15;
+    v *= 0x2C1B3C6Du;
+    return v ^ (v >> 13);
+}
+
+__global__ __launch_bounds__(kSmallThreads) void nm_small_kernel(const int4 *__restrict__ coords, int n, int q_rows,
+                                                                 KernelShape ks, Limits lim, uint32_t mask,
+                                                                 NbrHeader *__restrict__ h, int32_t *__restrict__ map)
+{
+    __shared__ int4 s_c[kSmallRows];
+    __shared__ uint32_t s_slot[kSmallSlots];
+    __shared__ int4 s_o[kSmallMaxK];
+    __shared__ int s_red[kSmallThreads / 64][kPartialInts];
+    __shared__ NbrHeader s_h;
+    __shared__ int s_dup, s_neg;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid == 0) s_dup = s_neg = 0;
+    if (tid < ks.K) {
+        int o[3];
+        offset_of(ks, tid, o);
+        s_o[tid] = make_int4(o[0], o[1], o[2], 0);
+    }
+    for (int i = tid; i <= (int)mask; i += kSmallThreads) s_slot[i] = 0xffffffffu;
+    __syncthreads();
+    int mn[4] = {INT_MAX, INT_MAX, INT_MAX, INT_MAX};
+    int mx[4] = {INT_MIN, INT_MIN, INT_MIN, INT_MIN};
+    bool neg = false;
+    for (int i = tid; i < n; i += kSmallThreads) {
+        const int4 c = coords[i];
+        s_c[i] = c;
+        const int v[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            mn[j] = min(mn[j], v[j]);
+            mx[j] = max(mx[j], v[j]);
+            neg |= v[j] < 0;
+        }
+    }
+    if (neg) s_neg = 1;
+    __syncthreads();
+    for (int i = tid; i < n; i += kSmallThreads) {
+        const int4 c = s_c[i];
+        uint32_t s = small_hash(c.x, c.y, c.z, c.w) & mask;
+        for (uint32_t probe = 0; probe <= mask; ++probe) {
+            const uint32_t old = atomicCAS(&s_slot[s], 0xffffffffu, (uint32_t)i);
+            if (old == 0xffffffffu) break;
+            if (same_coord(s_c[old], c)) {
+                atomicMin(&s_slot[s], (uint32_t)i);
+                s_dup = 1;
+                break;
+            }
+            s = (s + 1) & mask;
+        }
+    }
+    if (blockIdx.x == 0) {
+        // the header: bbox, negative flag, octree-order bits -> table plan
+        uint32_t uns = 0;
+        for (int i = tid; i < n; i += kSmallThreads)
+            if (i > 0) uns |= unsorted_levels(s_c[i - 1], s_c[i]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            mn[j] = wave_min_i32(mn[j]);
+            mx[j] = wave_max_i32(mx[j]);
+        }
+        uns = wave_or_u32(uns);
+        if (lane == 0) {
+            for (int j = 0; j < 4; ++j) {
+                s_red[wave][j] = mn[j];
+                s_red[wave][4 + j] = mx[j];
+            }
+            s_red[wave][8] = 0;
+            s_red[wave][9] = (int)uns;
+        }
+        __syncthreads();
+        if (tid < kPartialInts) {
+            int v = s_red[0][tid];
+            for (int w = 1; w < kSmallThreads / 64; ++w) v = reduce_partial(tid, v, s_red[w][tid]);
+            if (tid < 4)
+                s_h.bmin[tid] = v;
+            else if (tid < 8)
+                s_h.bmax[tid - 4] = v;
+            else if (tid == 8)
+                s_h.status = s_neg ? kStatusNegative : 0u;
+            else
+                s_h.unsorted = (uint32_t)v;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            const Plan p = make_plan(&s_h, lim);
+            s_h.plan = p;
+            s_h.mode = p.mode;
+            s_h.pad0 = 0;
+            if (p.mode == 4 && s_dup) s_h.status |= kStatusDupCell;
+        }
+        __syncthreads();
+        if (tid < (int)(sizeof(NbrHeader) / 16))
+            reinterpret_cast<uint4 *>(h)[tid] = reinterpret_cast<const uint4 *>(&s_h)[tid];
+    }
+    __syncthreads();
+    // The workgroup's rows, one (row, offset) entry per thread.  A coord past
+    // INT_MAX wraps to a negative one, which no row has (a set with one maps
+    // to -1 everywhere, as its build has no table).
+    const int row0 = blockIdx.x * kSmallQuery;
+    const int total = (min(row0 + kSmallQuery, q_rows) - row0) * ks.K;
+    for (int e = tid; e < total; e += kSmallThreads) {
+        const int r = e / ks.K, k = e - r * ks.K;
+        const int4 c = s_c[row0 + r], o = s_o[k];
+        const int4 q = make_int4(c.x, (int)((uint32_t)c.y + (uint32_t)o.x), (int)((uint32_t)c.z + (uint32_t)o.y),
+                                 (int)((uint32_t)c.w + (uint32_t)o.z));
+        int32_t found = SC_INVALID_NEIGHBOR_ROW;
+        if (!s_neg) {
+            uint32_t s = small_hash(q.x, q.y, q.z, q.w) & mask;
+            for (uint32_t probe = 0; probe <= mask; ++probe) {
+                const uint32_t v = s_slot[s];
+                if (v == 0xffffffffu) break;
+                if (same_coord(s_c[v], q)) {
+                    found = (int32_t)v;
+                    break;
+                }
+                s = (s + 1) & mask;
+            }
+        }
+        map[(int64_t)row0 * ks.K + e] = found;
+    }
+}
+
 }  // namespace
 }  // namespace sc
 
@@ -1013,6 +1159,15 @@ int sc_neighbor_map_build(const sc_conv_config *cfg, const int32_t *d_coords, in
         return SC_OK;
     }
     const int4 *c4 = (const int4 *)d_coords;
+    if (n_rows <= kSmallRows && K <= kSmallMaxK) {
+        uint32_t slots = 64;
+        while (slots < 4 * (uint32_t)n_rows) slots <<= 1;
+        const int64_t blocks = query_rows > 0 ? (query_rows + kSmallQuery - 1) / kSmallQuery : 1;
+        nm_small_kernel<<<(unsigned)blocks, kSmallThreads, 0, s>>>(c4, (int)n_rows, (int)query_rows, kernel_shape(cfg),
+                                                                   lim, slots - 1, h, d_map);
+        SC_LAUNCH_CHECK("nm_small_kernel launch");
+        return SC_OK;
+    }
     const unsigned bb = grid_for(n_rows, kBboxThreads, kBboxBlocks);
     nm_bbox_partial_kernel<<<bb, kBboxThreads, 0, s>>>(c4, n_rows, partials);
     SC_LAUNCH_CHECK("nm_bbox_partial_kernel launch");

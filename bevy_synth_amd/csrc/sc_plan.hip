@@ -781,6 +781,247 @@ __global__ __launch_bounds__(kThreads) void plan_fix_kernel(PlanArgs a)
     }
 }
 
+// The whole order in one launch (one workgroup), for at most kSmallRows query
+// rows: the seven kernels above are bound by their launches there (607 rows
+// 22.7 -> 7.2 us, 4,096 rows 24.0 -> 10.9; boxes beyond the grid 43 -> 10.9
+// and 56 -> 33).  Same modes, same order,
+// same header: rows in octree order keep theirs; else, when the 8^3-brick
+// cells of the bounding box fit an LDS bitmap (the largest grid such a plan
+// has), a row's position is the number of occupied cells before its own,
+// rows of duplicated coords following in row order; else a counting sort by
+// brick, rows in order inside one.
+constexpr int kSmallRows = 4096;
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWords = (1 << 20) / 32;  // bitmap words; or the brick counts (<= 8,192) and the rows by brick
+
+__device__ inline int small_scan_excl(int x, int *s_wave, int &total)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int inc = x;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(inc, off, 64);
+        if (lane >= off) inc += y;
+    }
+    __syncthreads();
+    if (lane == 63) s_wave[wave] = inc;
+    __syncthreads();
+    int before = 0;
+    total = 0;
+    for (int w = 0; w < kSmallThreads / 64; ++w) {
+        if (w < wave) before += s_wave[w];
+        total += s_wave[w];
+    }
+    return before + inc - x;
+}
+
+__global__ __launch_bounds__(kSmallThreads) void plan_small_order_kernel(PlanArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t s_bits[kSmallWords];
+    __shared__ uint32_t s_first[kSmallRows];  // lowest row of each occupied cell, by rank
+    __shared__ int s_part[kSmallThreads];
+    __shared__ int s_wave[kSmallThreads / 64];
+    __shared__ int s_red[kSmallThreads / 64][9];
+    __shared__ PlanHeader s_h;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = (int)a.n_q;
+    plan_init(a);
+    constexpr int kPer = kSmallRows / kSmallThreads;  // rows tid, tid + kSmallThreads, ...
+    int4 c[kPer];
+    int mn[4] = {INT_MAX, INT_MAX, INT_MAX, INT_MAX}, mx[4] = {INT_MIN, INT_MIN, INT_MIN, INT_MIN};
+    uint32_t uns = 0;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int i = tid + u * kSmallThreads;
+        if (i >= n) continue;
+        c[u] = a.coords[i];
+        const int v[4] = {c[u].x, c[u].y, c[u].z, c[u].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            mn[j] = min(mn[j], v[j]);
+            mx[j] = max(mx[j], v[j]);
+        }
+        if (i > 0) uns |= unsorted_levels(a.coords[i - 1], c[u]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        mn[j] = wave_min_i32(mn[j]);
+        mx[j] = wave_max_i32(mx[j]);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) uns |= __shfl_xor(uns, off, 64);
+    if (lane == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s_red[wave][j] = mn[j];
+            s_red[wave][4 + j] = mx[j];
+        }
+        s_red[wave][8] = (int)uns;
+    }
+    __syncthreads();
+    uns = 0;
+    for (int w = 0; w < kSmallThreads / 64; ++w) uns |= (uint32_t)s_red[w][8];
+    if (tid < 8) {
+        int r = s_red[0][tid];
+        for (int w = 1; w < kSmallThreads / 64; ++w) r = tid < 4 ? min(r, s_red[w][tid]) : max(r, s_red[w][tid]);
+        if (tid < 4)
+            s_h.bmin[tid] = a.hdr->bmin[tid] = r;
+        else
+            s_h.bmax[tid - 4] = a.hdr->bmax[tid - 4] = r;
+    }
+    __syncthreads();
+    const uint32_t deep = ((1u << kRankLevels) - 1u) & ~((1u << kOwnOrderLevels) - 1u);
+    if ((~uns & deep) != 0u) {
+        if (tid == 0) {
+            a.hdr->grid_mode = 2;
+            a.hdr->n_unique = n;
+        }
+        for (int i = tid; i < n; i += kSmallThreads) a.order[i] = i;
+        return;
+    }
+    const bool sorted = !(uns & 1u);
+    const GridGeom g = grid_geom(&s_h, sorted ? bitmap_cells(a) : a.grid_cap);
+    if (g.ok && g.cells <= 32 * kSmallWords) {
+        const int nw = (int)(g.cells / 32);
+        for (int i = tid; i < nw; i += kSmallThreads) s_bits[i] = 0u;
+        for (int i = tid; i < n; i += kSmallThreads) s_first[i] = 0xffffffffu;
+        __syncthreads();
+        int cell[kPer];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            if (tid + u * kSmallThreads >= n) continue;
+            cell[u] = (int)grid_cell(g, c[u]);
+            atomicOr(&s_bits[cell[u] >> 5], 1u << (cell[u] & 31));
+        }
+        __syncthreads();
+        // thread t owns `chunk` consecutive words (odd: distinct LDS banks)
+        const int chunk = ((nw + kSmallThreads - 1) / kSmallThreads) | 1;
+        const int w0 = min(tid * chunk, nw), w1 = min(w0 + chunk, nw);
+        int cnt = 0;
+        for (int w = w0; w < w1; ++w) cnt += __builtin_popcount(s_bits[w]);
+        int n_unique;
+        s_part[tid] = small_scan_excl(cnt, s_wave, n_unique);
+        __syncthreads();
+        int rank[kPer];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const int i = tid + u * kSmallThreads;
+            if (i >= n) continue;
+            const int w = cell[u] >> 5, t = w / chunk;
+            int r = s_part[t];
+            for (int v = t * chunk; v < w; ++v) r += __builtin_popcount(s_bits[v]);
+            rank[u] = r + __builtin_popcount(s_bits[w] & ((1u << (cell[u] & 31)) - 1u));
+        }
+        if (n_unique == n) {
+#pragma unroll
+            for (int u = 0; u < kPer; ++u)
+                if (tid + u * kSmallThreads < n) a.order[rank[u]] = tid + u * kSmallThreads;
+        } else {
+            // duplicated coords: each cell's lowest row takes its place, the
+            // others follow in row order
+#pragma unroll
+            for (int u = 0; u < kPer; ++u)
+                if (tid + u * kSmallThreads < n) atomicMin(&s_first[rank[u]], (uint32_t)(tid + u * kSmallThreads));
+            __syncthreads();
+            uint32_t *s_lead = s_bits;  // the bitmap is done with
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                const int i = tid + u * kSmallThreads;
+                if (i >= n) continue;
+                const bool lead = s_first[rank[u]] == (uint32_t)i;
+                if (lead) a.order[rank[u]] = i;
+                s_lead[i] = lead;
+            }
+            __syncthreads();
+            bool extra[kPer];  // kPer consecutive rows per thread
+            int ex = 0;
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                const int i = tid * kPer + u;
+                extra[u] = i < n && !s_lead[i];
+                ex += extra[u];
+            }
+            int n_extras;
+            int pos = n_unique + small_scan_excl(ex, s_wave, n_extras);
+#pragma unroll
+            for (int u = 0; u < kPer; ++u)
+                if (extra[u]) a.order[pos++] = tid * kPer + u;
+            if (tid == 0) a.hdr->n_extras = n_extras;
+        }
+        if (tid == 0) {
+            a.hdr->grid_mode = sorted ? 3 : 1;
+            a.hdr->brick_shift = 3;
+            a.hdr->n_bricks = (uint64_t)(g.cells / 512);
+            a.hdr->n_unique = n_unique;
+        }
+        return;
+    }
+    const BrickGrid b = brick_grid(&s_h, a.brick_cap);
+    if (tid == 0) {
+        a.hdr->brick_shift = b.shift;
+        a.hdr->n_bricks = b.total;
+    }
+    if (tid == 0 && sorted && g.ok) {
+        // the bitmap order past the LDS bitmap (1 M cells): bricks of 8^3, and
+        // sorted rows are in cell order inside one, so the sort gives it too
+        a.hdr->grid_mode = 3;
+        a.hdr->brick_shift = 3;
+        a.hdr->n_bricks = (uint64_t)(g.cells / 512);
+        a.hdr->n_unique = n;
+    }
+    if (b.shift < 0) {
+        for (int i = tid; i < n; i += kSmallThreads) a.order[i] = i;
+        return;
+    }
+    // counting sort by brick in LDS, each brick's rows then ranked by counting
+    // (four a read: a brick's rows start at a multiple of 4, padded with ~0;
+    // at most kSmallRows bricks hold rows, so 4 kSmallRows words suffice)
+    constexpr int kSeg = 4 * kSmallRows;
+    static_assert(2 * kSeg <= kSmallWords && kSeg <= 0xffff, "counts and rows fit the LDS array; 16-bit starts");
+    uint32_t *s_cnt = s_bits, *s_seg = s_bits + kSeg;
+    const int nb = (int)b.total;  // <= brick_cap <= 2 kSmallRows
+    for (int i = tid; i < nb; i += kSmallThreads) s_cnt[i] = 0u;
+    for (int i = tid; i < kSeg; i += kSmallThreads) s_seg[i] = 0xffffffffu;
+    __syncthreads();
+    int br[kPer], slot[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        if (tid + u * kSmallThreads >= n) continue;
+        br[u] = (int)brick_of(b, c[u]);
+        slot[u] = (int)atomicAdd(&s_cnt[br[u]], 1u);
+    }
+    __syncthreads();
+    // counts -> starts: in the order (high half) and in s_seg (low half)
+    auto both = [](uint32_t v) { return v << 16 | ((v + 3u) & ~3u); };
+    const int chunk = ((nb + kSmallThreads - 1) / kSmallThreads) | 1;
+    const int b0 = min(tid * chunk, nb), b1 = min(b0 + chunk, nb);
+    int cnt = 0, total;
+    for (int i = b0; i < b1; ++i) cnt += (int)both(s_cnt[i]);
+    uint32_t run = (uint32_t)small_scan_excl(cnt, s_wave, total);
+    for (int i = b0; i < b1; ++i) {
+        const uint32_t v = s_cnt[i];
+        s_cnt[i] = run;
+        run += both(v);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+        if (tid + u * kSmallThreads < n) s_seg[(s_cnt[br[u]] & 0xffffu) + slot[u]] = (uint32_t)(tid + u * kSmallThreads);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int i = tid + u * kSmallThreads;
+        if (i >= n) continue;
+        const uint32_t st = s_cnt[br[u]], en = br[u] + 1 < nb ? s_cnt[br[u] + 1] : (uint32_t)total;
+        int r = (int)(st >> 16);
+        for (uint32_t e = st & 0xffffu; e < (en & 0xffffu); e += 4) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(s_seg + e);
+            r += (v.x < (uint32_t)i) + (v.y < (uint32_t)i) + (v.z < (uint32_t)i) + (v.w < (uint32_t)i);
+        }
+        a.order[r] = i;
+    }
+}
+
 __device__ inline uint32_t slot_hash(int32_t v)
 {
     return ((uint32_t)v * 0x9E3779B1u) >> (32 - kHashBits);
@@ -1546,6 +1787,11 @@ int launch_plan_order(const PlanArgs &a, const PlanLayout &L, hipStream_t s)
     if (n_q == 0) {
         plan_init_kernel<<<grid_for(L.n_tiles * kPlanTileRows, kThreads, 1024), kThreads, 0, s>>>(a);
         SC_LAUNCH_CHECK("plan_init_kernel launch");
+        return SC_OK;
+    }
+    if (n_q <= kSmallRows) {
+        plan_small_order_kernel<<<1, kSmallThreads, 0, s>>>(a);
+        SC_LAUNCH_CHECK("plan_small_order_kernel launch");
         return SC_OK;
     }
     const unsigned nbb = grid_for(n_q, kThreads, kBboxBlocks);
