@@ -257,8 +257,8 @@ static int conv_forward_impl(const sc_conv_config *cfg, int act_dtype, const voi
         }
     }
     a.out = conv_out;
-    a.vec_out = (a.cout_g % 4 == 0) && (a.cout % 4 == 0) && ((uintptr_t)conv_out % 16 == 0) &&
-                ((uintptr_t)a.residual % 16 == 0) && (a.scatter_ch % 4 == 0);
+    const int64_t ch_all = a.cout_g | a.cout | a.scatter_ch;  // its low bits: what every count is a multiple of
+    a.vec_out = (uintptr_t)conv_out % 16 || (uintptr_t)a.residual % 16 ? 0 : (ch_all % 8 == 0 ? 8 : (ch_all % 4 == 0 ? 4 : 0));
     // The halo-staged path (bf16 activations, up to 27 offsets) reads the
     // plan; other shapes ignore it.
     if (d_plan && (uintptr_t)d_plan % 256 != 0)

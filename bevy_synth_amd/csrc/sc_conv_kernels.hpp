@@ -36,7 +36,7 @@ struct ConvArgs {
     int cin_g;
     int cout_g;
     int K;
-    int vec_out;      // 4-channel packed output stores allowed (counts and pointers aligned)
+    int vec_out;      // 4 or 8: packed output stores of that many channels allowed (counts and pointers aligned)
     // Fused epilogue (order: + bias -> LayerNorm over the row -> SiLU -> + residual).
     // LayerNorm needs every channel of a row in one workgroup (groups == 1, Cout <= 128).
     int ln;
@@ -205,6 +205,34 @@ struct Out4<_Float16> {
     }
 };
 
+// The same for 8 consecutive values, stored as whole 16-byte pieces.
+template <typename TO>
+struct Out8 {
+    typedef uint4 V;
+    static __device__ inline V pack(const float *v)
+    {
+        const uint2 a = Out4<TO>::pack(v), b = Out4<TO>::pack(v + 4);
+        return make_uint4(a.x, a.y, b.x, b.y);
+    }
+    static __device__ inline void unpack(const V &u, float *v)
+    {
+        Out4<TO>::unpack(make_uint2(u.x, u.y), v);
+        Out4<TO>::unpack(make_uint2(u.z, u.w), v + 4);
+    }
+};
+template <>
+struct Out8<float> {
+    struct V {
+        float4 a, b;
+    };
+    static __device__ inline V pack(const float *v) { return V{Out4<float>::pack(v), Out4<float>::pack(v + 4)}; }
+    static __device__ inline void unpack(const V &u, float *v)
+    {
+        Out4<float>::unpack(u.a, v);
+        Out4<float>::unpack(u.b, v + 4);
+    }
+};
+
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // One 16x16x32 MFMA step on 16-bit operands: bf16 (TA = uint16_t) or f16
@@ -282,6 +310,40 @@ __device__ inline void c2s_store4(const ConvArgs &a, const C2SRow &c, int64_t qr
         for (int cc = 0; cc < 4; ++cc)
             if (cc < nv) store_from_f32<TO>(out, base + cc, t[cc]);
     }
+}
+
+// c2s_store4 for 8 channels [col, col + 8), col a multiple of 8, child widths a
+// multiple of 8 (vec_out 8): one child row lookup and one 16-byte store.
+template <typename TO, bool kSharedSkip = true>
+__device__ inline void c2s_store8(const ConvArgs &a, const C2SRow &c, int64_t qrow, int col, const float *v)
+{
+    TO *out = static_cast<TO *>(a.out);
+    int64_t base;
+    if (a.scatter_rows) {
+        const int ch = a.scatter_shift >= 0 ? col >> a.scatter_shift : col / a.scatter_ch;
+        const int32_t r = a.scatter_rows[qrow * 8 + ch];
+        if (r < 0 || r >= a.scatter_n) return;
+        base = (int64_t)r * a.scatter_ch + (col - ch * a.scatter_ch);
+    } else {
+        base = qrow * a.cout + col;
+    }
+    float t[8];
+#pragma unroll
+    for (int cc = 0; cc < 8; ++cc) t[cc] = v[cc];
+    if (c.skip_row) {
+        const TO *pp = static_cast<const TO *>(c.skip_row);
+        if (kSharedSkip && a.skip_shift >= 2) {
+            // repeat factor >= 4: one parent value per 4 channels (the same one from 8 on)
+            const float s0 = load_as_f32<TO>(pp, col >> a.skip_shift), s1 = load_as_f32<TO>(pp, (col + 4) >> a.skip_shift);
+#pragma unroll
+            for (int cc = 0; cc < 8; ++cc) t[cc] += cc < 4 ? s0 : s1;
+        } else {
+#pragma unroll
+            for (int cc = 0; cc < 8; ++cc)
+                t[cc] += load_as_f32<TO>(pp, a.skip_shift >= 0 ? (col + cc) >> a.skip_shift : (col + cc) / a.skip_R);
+        }
+    }
+    *reinterpret_cast<typename Out8<TO>::V *>(out + base) = Out8<TO>::pack(t);
 }
 
 // ------------------------------------------------------ bf16 tile, v2
@@ -715,9 +777,13 @@ __global__ __launch_bounds__(kThreads, 2) void conv_v2_kernel(ConvArgs args)
 //
 // Tile = 256 rows x 128 output channels, 4 waves, two workgroups per CU;
 // wave w owns rows [128 (w/2), +128) x channels [64 (w%2), +64) as 8 x 4
-// blocks of v_mfma_f32_16x16x32_bf16 (transposed product: lane l ends with
-// channels 4*(l/16)+e of row l%16 of each block).  Stage = (32-channel chunk
-// c, used offset k), chunk-major.  Per stage a wave reads 8 operand fragments
+// blocks of v_mfma_f32_16x16x32_bf16 (transposed product: lane l holds four
+// channels of row l%16 of each block; the weight rows are dealt to the blocks
+// so that two blocks make 8 consecutive channels, one 16-byte store, residual
+// load or child-row lookup where channels 4*(l/16)+e of each block made two
+// of 8 bytes: the residual block of 1,040,679 x 128 1,700 -> 1,667 us, an int8
+// decoder stack 16.66 -> 16.40 ms).  Stage = (32-channel chunk c, used offset
+// k), chunk-major.  Per stage a wave reads 8 operand fragments
 // from the LDS halo (each feeds 4 MFMAs) and loads its 4 weight fragments
 // w[o, k, 32c..32c+32) from L2 straight into registers one stage ahead (the
 // two waves of a column half share them through L1), so stages need no
@@ -947,8 +1013,14 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
         const __amdgpu_buffer_rsrc_t w_rsrc =
             make_rsrc(static_cast<const char *>(args.wpack) + kPackHeaderBytes,
                       (uint32_t)((int64_t)args.cin / args.cin_g * n_ot) * w_tile_bytes);
+        // MFMA row m = 4 a + b of the lane's block j takes channel 32 (j / 2) + 8 a
+        // + 4 (j % 2) + b, so that a lane ends with 8 consecutive channels of
+        // a row per block pair (16-byte stores): lane l16 reads the fragment
+        // 2 (j / 2) + l16 / 8 at lane 8 ((l16 / 4) % 2) + 4 (j % 2) + l16 % 4
+        // (still 64 contiguous bytes per 4 lanes).
         const uint32_t w_lane = (uint32_t)(g * n_ot + (o0 >> 7)) * w_tile_bytes +
-                                (uint32_t)((o0 & 127) / 16 + 4 * ch) * kFrag + (uint32_t)(lane * kWLane);
+                                (uint32_t)((o0 & 127) / 16 + 4 * ch + (l16 >> 3)) * kFrag +
+                                (uint32_t)((8 * ((l16 >> 2) & 1) + (l16 & 3) + 16 * q4) * kWLane);
         const int n_halo_instr = (U + 15) >> 4;
 
         struct Cursor {
@@ -979,7 +1051,9 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
             const bool live = u.c < nkc;
             const uint32_t wk = w_lane + (uint32_t)((u.k * nkc + u.c) * 8) * kFrag;
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj) f[jj] = bload16(w_rsrc, live ? wk + (uint32_t)jj * kFrag : kOobOffset);
+            for (int jj = 0; jj < 4; ++jj)
+                f[jj] = bload16(w_rsrc, live ? wk + (uint32_t)(jj >> 1) * 2 * kFrag + (uint32_t)(jj & 1) * 4 * kWLane
+                                             : kOobOffset);
         };
         // Halo DMA: instruction wave + 4*ii fills halo rows 16*(wave + 4*ii) + lane/4;
         // the lane moves logical piece hslot(j, lane%4) of row j.  Issued as
@@ -1135,18 +1209,19 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
         __builtin_amdgcn_sched_barrier(0);
     }
 
-    // ---- epilogue: lane l holds channels oc0 + 16 j + 4 q4 + e of tile row
-    //      row0 + 16 i + l16; the lanes l16 + 16 m of the wave (kNT = 64) or
+    // ---- epilogue: lane l holds channels oc0 + 32 (j / 2) + 8 q4 + 4 (j % 2)
+    //      + e of tile row row0 + 16 i + l16 (8 consecutive ones per pair of
+    //      blocks, the 4 lanes of a row 64 bytes of 16-bit output); the lanes l16 + 16 m of the wave (kNT = 64) or
     //      of the two waves of a row half (kNT = 128) hold the whole row.
     TO *__restrict__ out = static_cast<TO *>(args.out);
     const TO *__restrict__ res = static_cast<const TO *>(args.residual);
-    const bool vec_ok = args.vec_out != 0;
+    const bool vec_ok = args.vec_out != 0, vec8 = args.vec_out >= 8;
     const int oc0 = o0 + 64 * ch;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int o = oc0 + j * 16 + 4 * q4 + e;
+            const int o = oc0 + 32 * (j >> 1) + 8 * q4 + 4 * (j & 1) + e;
             const bool ok = o < args.cout_g;
             const float bias = s_bias[o - o0], scale = s_scale[o - o0];
 #pragma unroll
@@ -1202,7 +1277,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
             for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int o = oc0 + j * 16 + 4 * q4 + e;
+                    const int o = oc0 + 32 * (j >> 1) + 8 * q4 + 4 * (j & 1) + e;
                     const float d = acc[i][j][e] - mean[i];
                     qv += o < args.cout_g ? d * d : 0.f;
                 }
@@ -1217,7 +1292,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int o = oc0 + j * 16 + 4 * q4 + e;
+                const int o = oc0 + 32 * (j >> 1) + 8 * q4 + 4 * (j & 1) + e;
                 const bool ok = o < args.cout_g;
                 const int og = o % args.ln_group;  // channel within the LayerNorm group
                 const float lw = (args.ln_w && ok) ? args.ln_w[og] : 1.f;
@@ -1243,15 +1318,24 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
             if (qrow[i] < 0) continue;
             const C2SRow crow = c2s_row<TO>(args, qrow[i]);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int oc = oc0 + j * 16 + 4 * q4;
+            for (int jp = 0; jp < 2; ++jp) {
+                const int oc = oc0 + 32 * jp + 8 * q4;
                 if (oc >= args.cout_g) continue;
-                float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+                float v[8];
+#pragma unroll
+                for (int cc = 0; cc < 8; ++cc) v[cc] = acc[i][2 * jp + (cc >> 2)][cc & 3];
                 if (args.silu) {
 #pragma unroll
-                    for (int cc = 0; cc < 4; ++cc) v[cc] = silu_f32(v[cc]);
+                    for (int cc = 0; cc < 8; ++cc) v[cc] = silu_f32(v[cc]);
                 }
-                c2s_store4<TO, !kLN>(args, crow, qrow[i], (int)(out_col0 + oc), min(4, args.cout_g - oc), v, vec_ok);
+                if (vec8) {
+                    c2s_store8<TO, !kLN>(args, crow, qrow[i], (int)(out_col0 + oc), v);
+                } else {
+                    c2s_store4<TO, !kLN>(args, crow, qrow[i], (int)(out_col0 + oc), min(4, args.cout_g - oc), v, vec_ok);
+                    if (oc + 4 < args.cout_g)
+                        c2s_store4<TO, !kLN>(args, crow, qrow[i], (int)(out_col0 + oc + 4), min(4, args.cout_g - oc - 4),
+                                             v + 4, vec_ok);
+                }
             }
             // one row block at a time: loads hoisted across blocks would
             // hold their registers beside the whole accumulator
@@ -1261,15 +1345,15 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
     }
 #pragma unroll
     for (int ih = 0; ih < kI; ih += kRG) {
-        typename Out4<TO>::V rv[kRG][4];
-        if (res && vec_ok) {
+        typename Out8<TO>::V rv[kRG][2];
+        if (res && vec8) {
 #pragma unroll
             for (int ii = 0; ii < kRG; ++ii)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int oc = oc0 + j * 16 + 4 * q4;
-                    if (qrow[ih + ii] >= 0 && oc + 3 < args.cout_g)
-                        rv[ii][j] = *reinterpret_cast<const typename Out4<TO>::V *>(
+                for (int jp = 0; jp < 2; ++jp) {
+                    const int oc = oc0 + 32 * jp + 8 * q4;
+                    if (qrow[ih + ii] >= 0 && oc < args.cout_g)
+                        rv[ii][jp] = *reinterpret_cast<const typename Out8<TO>::V *>(
                             res + (int64_t)qrow[ih + ii] * args.cout + out_col0 + oc);
                 }
         }
@@ -1279,28 +1363,45 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
             if (qrow[i] < 0) continue;
             const int64_t rowbase = (int64_t)qrow[i] * args.cout + out_col0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int oc = oc0 + j * 16 + 4 * q4;
-                float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            for (int jp = 0; jp < 2; ++jp) {
+                const int oc = oc0 + 32 * jp + 8 * q4;
+                if (oc >= args.cout_g) continue;
+                float v[8];
+#pragma unroll
+                for (int cc = 0; cc < 8; ++cc) v[cc] = acc[i][2 * jp + (cc >> 2)][cc & 3];
                 if (args.silu) {
 #pragma unroll
-                    for (int cc = 0; cc < 4; ++cc) v[cc] = silu_f32(v[cc]);
+                    for (int cc = 0; cc < 8; ++cc) v[cc] = silu_f32(v[cc]);
                 }
-                if (vec_ok && oc + 3 < args.cout_g) {
+                if (vec8) {
                     if (res) {
-                        float r4[4];
-                        Out4<TO>::unpack(rv[ii][j], r4);
+                        float r8[8];
+                        Out8<TO>::unpack(rv[ii][jp], r8);
 #pragma unroll
-                        for (int cc = 0; cc < 4; ++cc) v[cc] += r4[cc];
+                        for (int cc = 0; cc < 8; ++cc) v[cc] += r8[cc];
                     }
-                    *reinterpret_cast<typename Out4<TO>::V *>(out + rowbase + oc) = Out4<TO>::pack(v);
+                    *reinterpret_cast<typename Out8<TO>::V *>(out + rowbase + oc) = Out8<TO>::pack(v);
                 } else {
 #pragma unroll
-                    for (int cc = 0; cc < 4; ++cc) {
-                        if (oc + cc >= args.cout_g) continue;
-                        float t = v[cc];
-                        if (res) t += load_as_f32<TO>(res, rowbase + oc + cc);
-                        store_from_f32<TO>(out, rowbase + oc + cc, t);
+                    for (int h = 0; h < 8; h += 4) {
+                        if (vec_ok && oc + h + 3 < args.cout_g) {
+                            if (res) {
+                                float r4[4];
+                                Out4<TO>::unpack(
+                                    *reinterpret_cast<const typename Out4<TO>::V *>(res + rowbase + oc + h), r4);
+#pragma unroll
+                                for (int cc = 0; cc < 4; ++cc) v[h + cc] += r4[cc];
+                            }
+                            *reinterpret_cast<typename Out4<TO>::V *>(out + rowbase + oc + h) = Out4<TO>::pack(v + h);
+                            continue;
+                        }
+#pragma unroll
+                        for (int cc = h; cc < h + 4; ++cc) {
+                            if (oc + cc >= args.cout_g) continue;
+                            float t = v[cc];
+                            if (res) t += load_as_f32<TO>(res, rowbase + oc + cc);
+                            store_from_f32<TO>(out, rowbase + oc + cc, t);
+                        }
                     }
                 }
             }

@@ -149,7 +149,8 @@ def test_skinny_rows_edges(rows, cin, cout, dtype):
     assert_close(got, x.double().cpu().numpy() @ w.T.astype(np.float64) + b, TOL[torch.float32])
 
 
-@pytest.mark.parametrize("cout,form", [(1024, "plain"), (640, "residual")])
+# Cout a multiple of 8 (16-byte stores), of 4, of neither
+@pytest.mark.parametrize("cout,form", [(1024, "plain"), (640, "residual"), (1028, "residual"), (1030, "residual")])
 def test_halo_tiles_few_rows(oracle, cout, form):
     """Enough output channels that few rows stay on the halo-staged tiles:
     tiles over the LDS budget, mixed with others, and a partial last tile."""
