@@ -196,7 +196,7 @@ static int conv_forward_impl(const sc_conv_config *cfg, int act_dtype, const voi
     };
     a.scatter_shift = log2_or_neg(c2s.scatter_ch);
     a.skip_shift = log2_or_neg(c2s.skip_R);
-    a.tile_child = nullptr;
+    a.tile_child = a.child_base = nullptr;
     a.child_ch = (int)c2s.scatter_ch;
     a.child_plan = child_plan ? 1 : 0;
     if (c2s.scatter) a.ln_group = a.scatter_ch;

@@ -7,6 +7,7 @@
 #include "sc_common.hpp"
 #include "sc_plan.hpp"
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 namespace sc {
@@ -78,6 +79,7 @@ struct ConvArgs {
     // each belong to one child c, tile_child[t], and compute its output
     // channels [c * child_ch, (c + 1) * child_ch); child_plan marks the call.
     const int32_t *tile_child;
+    const int32_t *child_base;  // first list tile of each child (the persistent dense tile)
     int child_ch;
     int child_plan;
 };
@@ -1897,6 +1899,7 @@ __global__ __launch_bounds__(256) void conv_scalar_kernel(ConvArgs args)
 
 #include "sc_conv_rows.hpp"
 #include "sc_conv_f32.hpp"
+#include "sc_dense_tile.hpp"
 
 // 16-bit activations through the v2 tile: 128-byte stages when the group's
 // input channels allow it, else 64-byte stages with a deeper A prefetch.
@@ -2008,12 +2011,15 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                     h.plan_hdr = pv.hdr;
                     h.perm = pv.order;
                     h.tile_child = pv.tile_child;
+                    h.child_base = reinterpret_cast<const int32_t *>(static_cast<const char *>(plan) + CL.child_base);
                     if (const RowsCut cut = rows_cut(a.scatter_n, a.child_ch, 1); cut.kI) {
                         r.plan_hdr = pv.hdr;
                         r.perm = pv.order;
                         r.tile_child = pv.tile_child;
                         return launch_rows<TA, TW, TO>(r, cut, CL.n_main * kPlanTileRows, a.child_ch, 1, s);
                     }
+                    if (dense_tile_takes<TO>(a, true, (a.scatter_n + kTileRows - 1) / kTileRows))
+                        return launch_dense_tile<TA, TO, true>(h, CL.n_main, s);
                     const int64_t lgrid = CL.n_main * (a.child_ch / 128);
                     if (lgrid > INT32_MAX) return fail(SC_ERR_OVERFLOW, "dense linear grid overflow");
                     const dim3 lg((unsigned)lgrid, 1, 1);
@@ -2031,6 +2037,7 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                     SC_LAUNCH_CHECK("dense_gemm_kernel launch (child plan)");
                     return SC_OK;
                 }
+                if (dense_tile_takes<TO>(a, false, tiles)) return launch_dense_tile<TA, TO, false>(a, tiles, s);
                 if (wide_tile) {
                     if (staged)
                         dense_gemm_kernel<TA, TO, false, 4, sizeof(TO) == 2><<<dgrid, DenseShape<4>::kThreads, 0, s>>>(a);

@@ -1,0 +1,66 @@
+"""GPU tests of the persistent 256 x 256 tile of the dense linear
+(dense_tile_kernel, from 160 tiles on) at its edges: a last row tile of one row,
+a last column tile that is not full, the shortest ring (4 k-steps, 8 with child
+lists), one, two and five tiles per workgroup, f32 output, the epilogue's forms;
+child lists of very different lengths, one of them empty.
+
+Against the float64 product of the same rounded operands: bf16 / f16 outputs to
+half an ulp (2^-9, 2^-12 of the value; the bounds below leave a factor of two)
+plus the f32 sum's error; f32 outputs to 2e-5 (a sum of Cin <= 544 products in
+f32, whose error is near sqrt(Cin) 2^-24, about 2e-6)."""
+import numpy as np
+import pytest
+import torch
+
+from bevy_synth_amd import decoder as D
+from bevy_synth_amd import flex_gmm as F
+from tests.test_gpu_plan import dev
+from tests.test_gpu_small_tiles import TOL, shell
+from tests.tolerance import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+def randn(shape, seed, scale=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(shape, generator=g, device="cuda") * scale
+
+
+@pytest.mark.parametrize("rows,cin,cout,dtype,out,silu,residual", [
+    (10241, 128, 1024, torch.bfloat16, torch.bfloat16, False, False),  # 164 tiles, 4 k-steps
+    (10495, 128, 1024, torch.float16, torch.float32, True, True),      # 164, last row tile one row short
+    (20481, 160, 488, torch.bfloat16, torch.float32, False, True),     # 162, last column tile 232 wide
+    (40961, 192, 248, torch.float16, torch.float16, True, True),       # 161, 248 wide
+    (10241, 544, 2560, torch.bfloat16, torch.bfloat16, True, False),   # 410, above 512 channels
+    (70000, 128, 1024, torch.bfloat16, torch.bfloat16, False, True),   # 1,096: five rounds
+])
+def test_dense_tile_edges(rows, cin, cout, dtype, out, silu, residual):
+    x, w = randn((rows, cin), 1).to(dtype), randn((cout, cin), 2, cin ** -0.5).to(dtype)
+    b = randn((cout,), 3)
+    res = randn((rows, cout), 4).to(out) if residual else None
+    got = F.linear_forward(x, w, b, out_dtype=out, silu=silu, residual=res)
+    exp = x.double() @ w.double().T + b.double()
+    if silu:
+        exp = exp * torch.sigmoid(exp)
+    if residual:
+        exp = exp + res.double()
+    assert_close(got.double().cpu().numpy(), exp.cpu().numpy(), TOL[out], f"{rows} rows {cin}->{cout}")
+
+
+@pytest.mark.parametrize("n,cin,cout,dtype", [(20001, 256, 256, torch.bfloat16), (12000, 288, 512, torch.float16)])
+def test_dense_tile_child_lists(n, cin, cout, dtype):
+    """Children of 0 (always), 3 (never), 7 (one parent), the rest at random;
+    equal in every bit to the linear over all children."""
+    parents = dev(shell(n))
+    rng = np.random.default_rng(n)
+    on = rng.random((n, 8)) < [1, 0.2, 0.5, 0, 0.9, 0.5, 0.4, 0]
+    on[n - 1, 7] = True
+    mask = dev(on.astype(np.uint8))
+    x, w = randn((n, cin), 5).to(dtype), randn((8 * cout, cin), 6, cin ** -0.5).to(dtype)
+    layer = D.ConvLayer(F.SparseSubmConvConfig(cin, 8 * cout, 1, 1, 1), w.reshape(8 * cout, 1, cin),
+                        randn((8 * cout,), 7))
+    _, got, idx = D.transposed_upsample(parents, x, layer, mask)
+    _, every, _ = D.transposed_upsample(parents, x, layer, mask, active_only=False)
+    full = (x.double() @ w.double().T + layer.bias.double()).reshape(n * 8, cout)
+    assert_close(got.double().cpu().numpy(), full[torch.from_numpy(np.flatnonzero(on)).cuda()].cpu().numpy(), TOL[dtype])
+    assert torch.equal(got, every)
