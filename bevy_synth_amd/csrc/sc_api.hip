@@ -2,6 +2,7 @@
 // residual add, row gather, C2S skip add, dtype conversion) for gfx950.
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 
 #include "sc_common.hpp"
@@ -22,6 +23,68 @@ int fail(int status, const std::string &msg)
 int hip_fail(hipError_t err, const char *what)
 {
     return fail(SC_ERR_HIP, std::string(what) + ": " + hipGetErrorString(err));
+}
+
+// The header words that the checks read back go through pinned memory: a copy
+// into the caller's stack is staged by the runtime (map of 300,007 shuffled rows
+// with its check 79.7 us, so 72.6; the 607-row block 88 and 81).  One page of 64 words
+// for the process, a word held by one call at a time; with none free, or no
+// page, the copy goes to the stack.
+namespace {
+struct PinnedWords {
+    static constexpr int kWords = 64, kStride = 16;  // 64 bytes apart
+    std::mutex m;
+    uint32_t *page = nullptr;
+    uint64_t used = 0;
+    bool tried = false;
+    int take()
+    {
+        std::lock_guard<std::mutex> g(m);
+        if (!tried) {
+            tried = true;
+            // an allocation is refused while another thread captures a graph
+            // in the strict mode, and would end that capture
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            if (hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
+                void *q = nullptr;
+                if (hipHostMalloc(&q, kWords * kStride * sizeof(uint32_t), hipHostMallocPortable) == hipSuccess)
+                    page = static_cast<uint32_t *>(q);
+                (void)hipThreadExchangeStreamCaptureMode(&mode);
+            }
+            (void)hipGetLastError();
+        }
+        if (!page || used == ~0ull) return -1;
+        const int i = __builtin_ctzll(~used);
+        used |= 1ull << i;
+        return i;
+    }
+    void give(int i)
+    {
+        std::lock_guard<std::mutex> g(m);
+        used &= ~(1ull << i);
+    }
+};
+PinnedWords &pinned_words()
+{
+    static PinnedWords *w = new PinnedWords;  // lives until the process ends: calls may come from exit handlers
+    return *w;
+}
+}  // namespace
+
+int read_status(const uint32_t *d_word, uint32_t *value, hipStream_t s, const char *what)
+{
+    PinnedWords &words = pinned_words();
+    const int i = words.take();
+    uint32_t *dst = i >= 0 ? words.page + i * PinnedWords::kStride : value;
+    const hipError_t copied = hipMemcpyAsync(dst, d_word, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
+    const hipError_t synced = hipStreamSynchronize(s);  // in either case: the word is given back
+    if (i >= 0) {
+        *value = *dst;
+        words.give(i);
+    }
+    SC_HIP_CHECK(copied, what);
+    SC_HIP_CHECK(synced, what);
+    return SC_OK;
 }
 
 // validate_config, crates/burn_flex_gmm/src/lib.rs:698-725 (same messages).

@@ -17,6 +17,8 @@ void set_error(const std::string &msg);
 void clear_error();
 int fail(int status, const std::string &msg);
 int hip_fail(hipError_t err, const char *what);
+// Reads a 32-bit word of device memory after the work queued on s; waits for it.
+int read_status(const uint32_t *d_word, uint32_t *value, hipStream_t s, const char *what);
 
 #define SC_HIP_CHECK(expr, what)                                  \
     do {                                                          \

@@ -459,10 +459,9 @@ extern "C" int sc_conv_plan_check(const void *d_plan, sc_stream stream)
     if (!d_plan) return fail(SC_ERR_NULL, "conv plan buffer is NULL");
     hipStream_t s = as_stream(stream);
     uint32_t status = 0;
-    SC_HIP_CHECK(hipMemcpyAsync(&status, &static_cast<const PlanHeader *>(d_plan)->status, sizeof(status),
-                                hipMemcpyDeviceToHost, s),
-                 "conv plan status readback");
-    SC_HIP_CHECK(hipStreamSynchronize(s), "conv plan status sync");
+    if (const int rc = read_status(&static_cast<const PlanHeader *>(d_plan)->status, &status, s,
+                                   "conv plan status readback"))
+        return rc;
     if (status & kPlanStatusMapMismatch)
         return fail(SC_ERR_SHAPE, "sparse conv: the conv plan was built for another map (n_q, n_in or K differ); "
                                   "the conv wrote nothing");

@@ -1197,10 +1197,8 @@ int sc_neighbor_map_check(const void *d_workspace, sc_stream stream)
     if (!d_workspace) return fail(SC_ERR_NULL, "neighbor map workspace is NULL");
     hipStream_t s = as_stream(stream);
     uint32_t status = 0;
-    SC_HIP_CHECK(hipMemcpyAsync(&status, &((const NbrHeader *)d_workspace)->status, sizeof(status),
-                                hipMemcpyDeviceToHost, s),
-                 "neighbor map status readback");
-    SC_HIP_CHECK(hipStreamSynchronize(s), "neighbor map status sync");
+    if (const int rc = read_status(&((const NbrHeader *)d_workspace)->status, &status, s, "neighbor map status readback"))
+        return rc;
     if (status & kStatusNegative)
         return fail(SC_ERR_COORD, "coord value exceeds i32::MAX (negative i32) for device neighbor kernel");
     return SC_OK;

@@ -113,3 +113,35 @@ def test_small_map_edges_of_the_coord_range(oracle):
     assert (out == -1).all() and F.neighbor_map_table_mode(ws) == "none"
     with pytest.raises(F.SparseConvError):
         F.neighbor_map_check(ws)
+
+
+def test_status_words_of_several_threads():
+    """The checks of concurrent calls read their own status: only the threads
+    whose coords are negative are refused, on every repetition."""
+    import threading
+
+    cfg = F.SparseSubmConvConfig(32, 32)
+    wrong = []
+
+    def work(i):
+        c = torch.randint(0, 20, (500 + i, 4), dtype=torch.int32)
+        c[:, 0] = 0
+        if i % 2:
+            c[i, 1] = -1
+        with torch.cuda.stream(torch.cuda.Stream()):
+            c = c.cuda()
+            for _ in range(20):
+                try:
+                    F.neighbor_rows_tensor_from_coords_tensor(cfg, c)
+                    refused = False
+                except Exception:
+                    refused = True
+                if refused != bool(i % 2):
+                    wrong.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
