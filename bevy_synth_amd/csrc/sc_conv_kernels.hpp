@@ -779,11 +779,11 @@ __global__ __launch_bounds__(kThreads, 2) void conv_v2_kernel(ConvArgs args)
 //
 // Tile = 256 rows x 128 output channels, 4 waves, two workgroups per CU;
 // wave w owns rows [128 (w/2), +128) x channels [64 (w%2), +64) as 8 x 4
-// blocks of v_mfma_f32_16x16x32_bf16 (transposed product: lane l holds four
-// channels of row l%16 of each block; the weight rows are dealt to the blocks
-// so that two blocks make 8 consecutive channels, one 16-byte store, residual
-// load or child-row lookup where channels 4*(l/16)+e of each block made two
-// of 8 bytes: the residual block of 1,040,679 x 128 1,700 -> 1,667 us, an int8
+// blocks of v_mfma_f32_16x16x32_bf16 (transposed product: lane l holds
+// channels 4*(l/16)+e of row l%16 of each block; before the stores the lanes of
+// a row trade registers, so that two blocks make 8 consecutive channels, one
+// 16-byte store, residual load or child-row lookup where there were two of 8
+// bytes: the residual block of 1,040,679 x 128 1,700 -> 1,667 us, an int8
 // decoder stack 16.66 -> 16.40 ms).  Stage = (32-channel chunk c, used offset
 // k), chunk-major.  Per stage a wave reads 8 operand fragments
 // from the LDS halo (each feeds 4 MFMAs) and loads its 4 weight fragments
@@ -812,6 +812,17 @@ __global__ __launch_bounds__(kThreads, 2) void conv_v2_kernel(ConvArgs args)
 //
 // LDS: halo (960 + 1) x 64 B + source offsets 960 x 4 B + lmap 27 x 256 x 2 B
 // = 77 KB.
+// Channels 16 m + 4 q4 (m = 0: a, 1: b) of the 4 lanes q4 of an MFMA column ->
+// channels 8 q4 + 4 m: the bits (m, q4 / 2, q4 % 2) of a value's place rotate.
+__device__ inline void pair_to_row8(float &a, float &b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    const auto q = __builtin_amdgcn_permlane16_swap(r[0], r[1], false, false);
+    a = u2f(q[0]);
+    b = u2f(q[1]);
+}
+
 constexpr int kHaloK = 27;
 #ifndef SC_HALO_WS
 #define SC_HALO_WS 2
@@ -1015,14 +1026,8 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
         const __amdgpu_buffer_rsrc_t w_rsrc =
             make_rsrc(static_cast<const char *>(args.wpack) + kPackHeaderBytes,
                       (uint32_t)((int64_t)args.cin / args.cin_g * n_ot) * w_tile_bytes);
-        // MFMA row m = 4 a + b of the lane's block j takes channel 32 (j / 2) + 8 a
-        // + 4 (j % 2) + b, so that a lane ends with 8 consecutive channels of
-        // a row per block pair (16-byte stores): lane l16 reads the fragment
-        // 2 (j / 2) + l16 / 8 at lane 8 ((l16 / 4) % 2) + 4 (j % 2) + l16 % 4
-        // (still 64 contiguous bytes per 4 lanes).
         const uint32_t w_lane = (uint32_t)(g * n_ot + (o0 >> 7)) * w_tile_bytes +
-                                (uint32_t)((o0 & 127) / 16 + 4 * ch + (l16 >> 3)) * kFrag +
-                                (uint32_t)((8 * ((l16 >> 2) & 1) + (l16 & 3) + 16 * q4) * kWLane);
+                                (uint32_t)((o0 & 127) / 16 + 4 * ch) * kFrag + (uint32_t)(lane * kWLane);
         const int n_halo_instr = (U + 15) >> 4;
 
         struct Cursor {
@@ -1053,9 +1058,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
             const bool live = u.c < nkc;
             const uint32_t wk = w_lane + (uint32_t)((u.k * nkc + u.c) * 8) * kFrag;
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj)
-                f[jj] = bload16(w_rsrc, live ? wk + (uint32_t)(jj >> 1) * 2 * kFrag + (uint32_t)(jj & 1) * 4 * kWLane
-                                             : kOobOffset);
+            for (int jj = 0; jj < 4; ++jj) f[jj] = bload16(w_rsrc, live ? wk + (uint32_t)jj * kFrag : kOobOffset);
         };
         // Halo DMA: instruction wave + 4*ii fills halo rows 16*(wave + 4*ii) + lane/4;
         // the lane moves logical piece hslot(j, lane%4) of row j.  Issued as
@@ -1211,10 +1214,10 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
         __builtin_amdgcn_sched_barrier(0);
     }
 
-    // ---- epilogue: lane l holds channels oc0 + 32 (j / 2) + 8 q4 + 4 (j % 2)
-    //      + e of tile row row0 + 16 i + l16 (8 consecutive ones per pair of
-    //      blocks, the 4 lanes of a row 64 bytes of 16-bit output); the lanes l16 + 16 m of the wave (kNT = 64) or
-    //      of the two waves of a row half (kNT = 128) hold the whole row.
+    // ---- epilogue: lane l holds channels oc0 + 16 j + 4 q4 + e of tile row
+    //      row0 + 16 i + l16 (LayerNorm's sums add in this order, the same
+    //      as the dense kernels'); the lanes l16 + 16 m of the wave (kNT = 64)
+    //      or of the two waves of a row half (kNT = 128) hold the whole row.
     TO *__restrict__ out = static_cast<TO *>(args.out);
     const TO *__restrict__ res = static_cast<const TO *>(args.residual);
     const bool vec_ok = args.vec_out != 0, vec8 = args.vec_out >= 8;
@@ -1223,7 +1226,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
     for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int o = oc0 + 32 * (j >> 1) + 8 * q4 + 4 * (j & 1) + e;
+            const int o = oc0 + j * 16 + 4 * q4 + e;
             const bool ok = o < args.cout_g;
             const float bias = s_bias[o - o0], scale = s_scale[o - o0];
 #pragma unroll
@@ -1279,7 +1282,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
             for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int o = oc0 + 32 * (j >> 1) + 8 * q4 + 4 * (j & 1) + e;
+                    const int o = oc0 + j * 16 + 4 * q4 + e;
                     const float d = acc[i][j][e] - mean[i];
                     qv += o < args.cout_g ? d * d : 0.f;
                 }
@@ -1294,7 +1297,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int o = oc0 + 32 * (j >> 1) + 8 * q4 + 4 * (j & 1) + e;
+                const int o = oc0 + j * 16 + 4 * q4 + e;
                 const bool ok = o < args.cout_g;
                 const int og = o % args.ln_group;  // channel within the LayerNorm group
                 const float lw = (args.ln_w && ok) ? args.ln_w[og] : 1.f;
@@ -1304,6 +1307,21 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
                 __builtin_amdgcn_sched_barrier(0);
             }
     }
+    // The stores want 8 consecutive channels a lane (16 bytes, the 4 lanes of
+    // a row 64): lane q4 = 2 q1 + q0 trades registers with its row's other
+    // lanes until block pair jp holds channels oc0 + 32 jp + 8 q4 + [0, 8).
+    // 16 instructions per row block, once a tile; every lane takes part.
+#pragma unroll
+    for (int i = 0; i < kI; ++i)
+#pragma unroll
+        for (int jp = 0; jp < 2; ++jp)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float a = acc[i][2 * jp][e], b = acc[i][2 * jp + 1][e];
+                pair_to_row8(a, b);
+                acc[i][2 * jp][e] = a;
+                acc[i][2 * jp + 1][e] = b;
+            }
     // Stores: the residual of kRG row blocks (4 for bf16, 2 for f32 outputs)
     // is fetched before any of them is written, so its latency overlaps
     // instead of serialising per block.

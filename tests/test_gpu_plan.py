@@ -352,6 +352,27 @@ def test_planned_ln_silu_and_residual(oracle, affine, cin, cout):
     assert_close(out2.cpu().numpy(), exp2, 2e-5, "planned residual")
 
 
+@pytest.mark.parametrize("cout", [40, 64, 100, 128])  # 64- and 128-channel tiles, full and not
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_planned_layer_norm_sums_as_the_linear(cout, dtype):
+    """A planned 1x1x1 conv and the linear on the same operands (40,000 rows:
+    the halo-staged and the dense tiles) form the same sums, those of
+    LayerNorm included: the f32 outputs agree in every bit."""
+    rng = np.random.default_rng(cout)
+    n, cin = 40000, 96
+    c = synth.config2_coords()[:n]
+    cfg = F.SparseSubmConvConfig(cin, cout, 1, 1, 1)
+    cd = dev(c)
+    nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, cd)
+    x = dev(synth.normal_f32(rng, (n, cin))).to(dtype)
+    w = dev(synth.conv_weight(rng, cout, 1, cin, 0.1)).to(dtype)
+    b, lw, lb = (dev(synth.normal_f32(rng, cout)) for _ in range(3))
+    kw = dict(layer_norm=True, ln_weight=lw, ln_bias=lb, silu=True, out_dtype=torch.float32)
+    conv = F.sparse_subm_conv_forward(cfg, x, nbr, w, b, plan=F.build_conv_plan(cfg, cd, nbr),
+                                      packed_weight=F.pack_conv_weight(cfg, w), **kw)
+    assert torch.equal(conv, F.linear_forward(x, w.reshape(cout, cin), b, **kw))
+
+
 def spread_neighbour_coords(spacing, far=0):
     """One tile of 256 query centres (batch 0, x = 3i), each with two
     neighbours ((3i+1, 0, 0) and (3i, 1, 0)) stored `spacing` rows apart after
