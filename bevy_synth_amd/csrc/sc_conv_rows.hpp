@@ -12,11 +12,14 @@
 // of the input rows at one offset; its operands (kI row slices, 4 weight
 // fragments, one 16-byte load per lane each) are loaded kDepth - 1 stages
 // ahead straight into registers: LDS holds only the rows' neighbour offsets.
-// kSplit waves of the workgroup share a block, each taking every kSplit-th
-// stage, and add their partial sums through LDS: a 27-offset conv of 64
-// channels is 54 stages, which one wave would run one after the other.  The
-// other waves take the 64-channel columns of the kNT-channel tile, then row
-// blocks.  A wave walks only the offsets that its own rows use.
+// kSplit waves of the workgroup share a block, wave s taking offset k of chunk
+// c when (k + c) % kSplit == s, and add their partial sums through LDS: a
+// 27-offset conv of 64 channels is 54 stages, which one wave would run one
+// after the other.  The other waves take the 64-channel columns of the
+// kNT-channel tile, then row blocks.  A wave walks only the offsets that its
+// own rows use; the deal goes by the offset itself and not by its place in
+// that list, so that a row's value does not depend on which rows share its
+// block.
 //
 // Bound, measured: the load path, 16 bytes a lane from 16 different rows
 // taking 64 cycles a fragment (packed weights, whole lines per 4 lanes, 16),
@@ -60,7 +63,7 @@ __global__ __launch_bounds__(kThreads, kI == 1 ? 3 : 2) void conv_rows_kernel(Co
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, q4 = lane >> 4;
-    const int sp = wave % kSplit;                   // the wave's share of the stages
+    const int sp = __builtin_amdgcn_readfirstlane(wave) % kSplit;  // the wave's share of the stages
     const int ch = wave / kSplit % T::kColWaves;    // its 64 channels
     const int rw = wave / (kSplit * T::kColWaves);  // and its row blocks
     const int trow = 16 * kI * rw;                  // first tile row of the wave
@@ -152,9 +155,12 @@ __global__ __launch_bounds__(kThreads, kI == 1 ? 3 : 2) void conv_rows_kernel(Co
 
     const int oc0 = o0 + 64 * ch;
     const int nkc = args.cin_g / kEl;
-    // the wave's stages: sp, sp + kSplit, ... of the list
-    const int S_all = __builtin_popcount(wmask) * nkc;
-    const int S = S_all > sp ? (S_all - sp + kSplit - 1) / kSplit : 0;
+    // the wave's offsets in chunk c, and its stages over all chunks
+    constexpr uint32_t kDeal = kSplit == 4 ? 0x11111111u : (kSplit == 2 ? 0x55555555u : 0xffffffffu);
+    auto share = [&](int c) { return wmask & (kDeal << ((sp - c) & (kSplit - 1))); };
+    int S = 0;
+#pragma unroll
+    for (int c = 0; c < kSplit; ++c) S += __builtin_popcount(share(c)) * ((nkc - c + kSplit - 1) / kSplit);
     if (S > 0) {
         const __amdgpu_buffer_rsrc_t a_rsrc =
             make_rsrc(static_cast<const TA *>(args.input) + in_col0,
@@ -187,16 +193,12 @@ __global__ __launch_bounds__(kThreads, kI == 1 ? 3 : 2) void conv_rows_kernel(Co
             }
         }
         const uint32_t *offs = &s_off[0][trow + l16];
-        uint32_t rem = wmask;   // offsets left in the chunk of the next stage to load
+        uint32_t rem = share(0);  // offsets left in the chunk of the next stage to load
         int c = 0;
-        auto next = [&]() {
-            rem &= rem - 1u;
-            if (rem == 0u) {
-                rem = wmask;
-                ++c;
-            }
+        auto settle = [&]() {  // past the last chunk: offset 0, never loaded
+            while (rem == 0u) rem = ++c < nkc ? share(c) : 1u;
         };
-        for (int u = 0; u < sp; ++u) next();
+        settle();
         int k = __builtin_ctz(rem);
         uint32_t ro[kI];
         auto read_off = [&]() {
@@ -221,8 +223,8 @@ __global__ __launch_bounds__(kThreads, kI == 1 ? 3 : 2) void conv_rows_kernel(Co
                     w[s][j] = bload16(w_rsrc, off);
                 }
             }
-#pragma unroll
-            for (int u = 0; u < kSplit; ++u) next();
+            rem &= rem - 1u;
+            settle();
             k = __builtin_ctz(rem);
             read_off();
         };

@@ -106,6 +106,26 @@ def test_rows_tile_forms(oracle, dtype, w, cin, cout, groups, ln, out, n, planne
     conv_case(oracle, n, cin, cout, dtype, w, planned, ln, not ln, groups, out)
 
 
+@pytest.mark.parametrize("cin,cout,ln", [(32, 64, False), (96, 128, True), (64, 200, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_tile_row_alone(cin, cout, ln, dtype):
+    """A row's value, in every bit, is the one it has with no other row using
+    any offset: which rows share its block does not enter its sum."""
+    n = 90
+    rng = np.random.default_rng(cin)
+    nbr = np.where(rng.random((n, 27)) < 0.4, -1, rng.integers(0, n, (n, 27))).astype(np.int32)
+    x, w = dev(synth.normal_f32(rng, (n, cin))).to(dtype), dev(synth.conv_weight(rng, cout, 27, cin, 0.05)).to(dtype)
+    cfg = F.SparseSubmConvConfig(cin, cout)
+
+    def conv(m):
+        return F.sparse_subm_conv_forward(cfg, x, dev(m), w, layer_norm=ln, out_dtype=torch.float32)
+    together = conv(nbr)
+    for r in (0, 17, n - 1):
+        alone = np.full_like(nbr, -1)
+        alone[r] = nbr[r]
+        assert torch.equal(conv(alone)[r], together[r]), r
+
+
 @pytest.mark.parametrize("n,cin,cout,groups,ln,kernel,out", [
     (1, 16, 64, 1, False, (3, 3, 3), None),
     (31, 16, 24, 1, True, (3, 3, 3), None),
