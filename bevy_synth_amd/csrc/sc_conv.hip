@@ -107,6 +107,12 @@ static bool ln_in_tile(const sc_conv_config *cfg, int act_dtype, const C2SForms 
     return cfg->out_channels_per_group <= kBN;
 }
 
+static bool ranges_overlap(const void *a, int64_t a_bytes, const void *b, int64_t b_bytes)
+{
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return a && b && x < y + (uintptr_t)b_bytes && y < x + (uintptr_t)a_bytes;
+}
+
 // dense: the linear layer (a 1x1x1 kernel without a map: query row r reads
 // input row r).
 static int conv_forward_impl(const sc_conv_config *cfg, int act_dtype, const void *d_input,
@@ -218,9 +224,13 @@ static int conv_forward_impl(const sc_conv_config *cfg, int act_dtype, const voi
     // kernel applies LayerNorm -> SiLU -> + residual and rounds once.
     // An f32 conv with an f32 output (which needs no workspace) also takes
     // the row kernel when a tile as wide as the row would leave the chip idle
-    // (the row kernel's 4-15 us against a conv of twice the time or more).
+    // (the row kernel's 4-15 us against a conv of twice the time or more), but
+    // not where the accumulators in d_out would overwrite the residual: the
+    // tile's lanes read their residual before they store.
     bool row_fuse = mfma && ln_in_tile(cfg, act_dtype, c2s);
+    const int64_t out_bytes = n_q * cfg->out_channels * (int64_t)dtype_size(out_dtype);
     if (row_fuse && act_f32 && out_dtype == SC_DTYPE_F32 && !c2s.skip &&
+        !ranges_overlap(d_residual, out_bytes, d_out, out_bytes) &&
         f32_tile(n_q, a.cout_g, groups) < f32_row_tile(a.cout_g)) {
         const int64_t t = 32 * f32_row_tile(a.cout_g);
         if ((n_q + t - 1) / t < 224) row_fuse = false;

@@ -210,12 +210,15 @@ typedef struct sc_conv_epilogue {
  * kernel, on the f32 accumulators, for every shape; so does LayerNorm when
  * one workgroup holds whole rows (groups == 1, Cout <= 128, the MFMA tile:
  * Cin_g a multiple of 32 (bf16) / 16 (f32), K <= 32, 16-byte aligned
- * pointers).  Otherwise the conv stores its f32 accumulators -- into d_out
+ * pointers), except that an f32 call of few rows may stage them.  Otherwise
+ * the conv stores its f32 accumulators -- into d_out
  * for an f32 output, else into epi->workspace (n_q * Cout * 4 bytes; without
  * it the call fails with SC_ERR_WORKSPACE) -- and one stream-ordered row
  * kernel applies LayerNorm -> SiLU -> + residual to them (the reference
  * normalises its f32 conv output the same way, sparse_decoder_wgpu_ops.rs
- * :1642-1711). */
+ * :1642-1711).  d_out may be the residual itself (same address), except where
+ * an f32 output stages a LayerNorm that one workgroup cannot hold: the
+ * accumulators then overwrite it. */
 int sc_subm_conv_forward_fused(const sc_conv_config *cfg, int act_dtype, const void *d_input,
                                int64_t n_in, const int32_t *d_map, int64_t n_q, int w_dtype,
                                const void *d_weight, const float *d_w_scale, const float *d_bias,

@@ -145,6 +145,34 @@ def test_f32_tile_edges(oracle, n, cin, cout, groups, ln, kernel, out):
               rows=lambda q: np.unique(np.r_[0:min(q, 400), max(0, q - 400):q]))
 
 
+# on both sides of the row counts up to which f32 stages a LayerNorm's rows
+# through the output
+@pytest.mark.parametrize("n,c", [(600, 64), (12288, 64), (12289, 64), (600, 128), (28544, 128), (28545, 128)])
+@pytest.mark.parametrize("linear", [False, True])
+def test_f32_layer_norm_residual_in_place(n, c, linear):
+    """The output may be the residual's own buffer."""
+    rng = np.random.default_rng(n + c)
+    x, b, res = (dev(synth.normal_f32(rng, s)) for s in ((n, c), (c,), (n, c)))
+    kw = dict(layer_norm=True, silu=True)
+    if linear:
+        w = dev(synth.normal_f32(rng, (c, c), 0.1))
+
+        def call(r, out):
+            return F.linear_forward(x, w, b, residual=r, out=out, **kw)
+    else:
+        cfg = F.SparseSubmConvConfig(c, c)
+        nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, dev(shell(n)))
+        w = dev(synth.conv_weight(rng, c, 27, c, 0.05))
+
+        def call(r, out):
+            return F.sparse_subm_conv_forward(cfg, x, nbr, w, b, residual=r, out=out, **kw)
+    apart, buf = call(res, None), res.clone()
+    call(buf, buf)
+    # one sum order either way; the row kernel and the tile add LayerNorm's
+    # statistics in different orders
+    assert_close(buf.cpu().numpy(), apart.cpu().numpy(), 4e-5)
+
+
 def test_f32_tile_isolated_rows(oracle):
     """Rows without any neighbour but one offset, and a map of -1 only."""
     cfg = F.SparseSubmConvConfig(16, 48)
