@@ -336,7 +336,7 @@ template <typename TO>
 int launch_f32(const ConvArgs &a, int groups, hipStream_t s)
 {
     int kB = f32_tile(a.n_q, a.cout_g, groups);
-    if (a.ln) kB = std::max(kB, f32_row_tile(a.cout_g));
+    if (a.ln || a.in_place) kB = std::max(kB, f32_row_tile(a.cout_g));
     while (kB < 4 && (a.cout_g + 32 * kB - 1) / (32 * kB) > 65535) kB *= 2;
     const int64_t gx = (a.n_q + 32 * kB - 1) / (32 * kB), gy = (a.cout_g + 32 * kB - 1) / (32 * kB);
     if (gx > INT32_MAX || gy > 65535 || groups > 65535) return fail(SC_ERR_OVERFLOW, "sparse conv grid overflow");

@@ -82,6 +82,12 @@ struct ConvArgs {
     const int32_t *child_base;  // first list tile of each child (the persistent dense tile)
     int child_ch;
     int child_plan;
+    // The output overlaps the input (host only).  A linear whose row's output
+    // channels lie in one tile (at most 128; 256 on 16-bit weights without
+    // LayerNorm) may write over its input: a workgroup then reads only rows
+    // that it alone writes, all of them before it stores.  Such calls stay off
+    // the smaller tiles, whose column tiles are workgroups of their own.
+    int in_place;
 };
 
 // The f32 tile (conv_f32_kernel): 16-row blocks per wave and side, a workgroup
@@ -1977,7 +1983,8 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                 // a child plan is sized by a bound on the children, of which
                 // about half are active
                 const int64_t rows = a.child_plan ? n_tiles * kPlanTileRows : a.n_q;
-                if (const RowsCut cut = rows_cut(a.child_plan ? a.scatter_n / 2 : rows, cols, groups); cut.kI) {
+                if (const RowsCut cut = rows_cut(a.child_plan ? a.scatter_n / 2 : rows, cols, groups);
+                    cut.kI && !a.in_place) {
                     r.plan_hdr = pv.hdr;
                     if (a.child_plan) {
                         r.tile_child = pv.tile_child;
@@ -2012,7 +2019,7 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                 const int64_t ncol = (a.cout_g + (wide_tile ? 255 : 127)) / (wide_tile ? 256 : 128);
                 if (tiles * ncol > INT32_MAX) return fail(SC_ERR_OVERFLOW, "dense linear grid overflow");
                 if (!a.child_plan)
-                    if (const RowsCut cut = rows_cut(a.n_q, a.cout_g, 1); cut.kI)
+                    if (const RowsCut cut = rows_cut(a.n_q, a.cout_g, 1); cut.kI && !a.in_place)
                         return launch_rows<TA, TW, TO>(r, cut, a.n_q, a.cout_g, 1, s);
                 const dim3 dgrid((unsigned)(tiles * ncol), 1, 1);
                 // row-contiguous stores through LDS: 16-bit output, 8-channel
@@ -2074,7 +2081,7 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                 }
                 SC_LAUNCH_CHECK("dense_gemm_kernel launch");
             } else {
-                if (const RowsCut cut = rows_cut(a.n_q, a.cout_g, groups); cut.kI)
+                if (const RowsCut cut = rows_cut(a.n_q, a.cout_g, groups); cut.kI && !a.in_place)
                     return launch_rows<TA, TW, TO>(r, cut, a.n_q, a.cout_g, groups, s);
                 launch_v2<TA, TW, TO>(a, grid, s);
             }

@@ -248,6 +248,10 @@ int sc_conv_epilogue_workspace_size(const sc_conv_config *cfg, int act_dtype, in
  * out_channels = 8 x C, and slice c of row r lands in row child_rows[r * 8 +
  * c] of an [n_child_rows][C] output (LayerNorm, when asked, per child);
  * epi->skip_index, the conv2 form, is refused.
+ * On the MFMA tile, d_out may be the input itself (in_channels ==
+ * out_channels, one type) when out_channels <= 128, or <= 256 with 16-bit
+ * weights and no LayerNorm; wider rows are written by several workgroups, and
+ * their output must not overlap the input.
  */
 int sc_linear_forward(int act_dtype, const void *d_input, int64_t rows, int64_t in_channels,
                       int64_t out_channels, int w_dtype, const void *d_weight, const float *d_w_scale,

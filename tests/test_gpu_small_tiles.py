@@ -173,6 +173,29 @@ def test_f32_layer_norm_residual_in_place(n, c, linear):
     assert_close(buf.cpu().numpy(), apart.cpu().numpy(), 4e-5)
 
 
+@pytest.mark.parametrize("n,c,dtype,w8,ln", [
+    (300, 64, torch.float32, False, False), (6001, 128, torch.float32, False, False),
+    (60000, 128, torch.float32, False, False), (600, 128, torch.float32, False, True),
+    (300, 128, torch.bfloat16, False, True), (3000, 256, torch.float16, False, False),
+    (45000, 256, torch.bfloat16, False, False),   # 176 tiles of 256 x 256
+    (5000, 128, torch.bfloat16, True, False)])
+def test_linear_over_its_input(n, c, dtype, w8, ln):
+    """A linear whose row of output channels lies in one tile may write over
+    its input, whatever the number of rows."""
+    rng = np.random.default_rng(n)
+    x = dev(synth.normal_f32(rng, (n, c))).to(dtype)
+    w, b, scale = dev(synth.normal_f32(rng, (c, c), 0.1)).to(dtype), dev(synth.normal_f32(rng, c)), None
+    if w8:
+        q, scale = synth.int8_weight(rng, c, 1, c)
+        w, scale = dev(q.reshape(c, c)), dev(scale)
+    exp = x.double() @ (w.double() * (scale[:, None] if w8 else 1)).T + b.double()
+    if ln:
+        exp = torch.nn.functional.layer_norm(exp, (c,), eps=1e-6)
+    buf = x.clone()
+    assert F.linear_forward(buf, w, b, scale, layer_norm=ln, out=buf, out_dtype=dtype) is buf
+    assert_close(buf.double().cpu().numpy(), exp.cpu().numpy(), max(TOL[dtype], 4e-5))
+
+
 def test_f32_tile_isolated_rows(oracle):
     """Rows without any neighbour but one offset, and a map of -1 only."""
     cfg = F.SparseSubmConvConfig(16, 48)
