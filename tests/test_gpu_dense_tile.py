@@ -47,7 +47,11 @@ def test_dense_tile_edges(rows, cin, cout, dtype, out, silu, residual):
     assert_close(got.double().cpu().numpy(), exp.cpu().numpy(), TOL[out], f"{rows} rows {cin}->{cout}")
 
 
-@pytest.mark.parametrize("n,cin,cout,dtype", [(20001, 256, 256, torch.bfloat16), (12000, 288, 512, torch.float16)])
+@pytest.mark.parametrize("n,cin,cout,dtype", [
+    (20001, 256, 256, torch.bfloat16), (12000, 288, 512, torch.float16),
+    # the row-block tile's limit of 2,048 blocks over all children, and lists
+    # that stay below it past that
+    (1024, 256, 256, torch.bfloat16), (1025, 256, 256, torch.bfloat16), (3900, 64, 128, torch.float16)])
 def test_dense_tile_child_lists(n, cin, cout, dtype):
     """Children of 0 (always), 3 (never), 7 (one parent), the rest at random;
     equal in every bit to the linear over all children."""
