@@ -1980,10 +1980,17 @@ int launch_conv(const ConvArgs &a, int groups, bool mfma, const void *plan, hipS
                 h.plan_hdr = pv.hdr;
                 h.tile_child = pv.tile_child;
                 if (sizeof(TW) != 1) h.w_scale = nullptr;
-                // a child plan is sized by a bound on the children, of which
-                // about half are active
+                // A child plan is sized by a bound on the children, of which
+                // half to three quarters are active.  The row blocks' time
+                // doubles where their workgroups no longer fit at once:
+                // children of 128 and more gain up to there and lose 4 % past
+                // it (3,250 parents x 128: half active 64 us against 105, three
+                // quarters 112 against 106), so half is counted; children of
+                // 64 gain less and lose 20 % (6,500 parents: 36 and 52 us
+                // against 42), so three quarters are.
                 const int64_t rows = a.child_plan ? n_tiles * kPlanTileRows : a.n_q;
-                if (const RowsCut cut = rows_cut(a.child_plan ? a.scatter_n / 2 : rows, cols, groups);
+                const int64_t active = cols <= 64 ? a.scatter_n / 4 * 3 : a.scatter_n / 2;
+                if (const RowsCut cut = rows_cut(a.child_plan ? active : rows, cols, groups);
                     cut.kI && !a.in_place) {
                     r.plan_hdr = pv.hdr;
                     if (a.child_plan) {

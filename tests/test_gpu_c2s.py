@@ -361,20 +361,24 @@ def test_child_plan_lists(frac):
     F.conv_plan_check(cp)
 
 
-@pytest.mark.parametrize("cin,cchild,ln", [(128, 64, True), (256, 128, True), (128, 256, True),
-                                           (128, 64, False)])
-def test_conv1_child_plan_matches_parent_plan(cin, cchild, ln):
+@pytest.mark.parametrize("cin,cchild,ln,n", [(128, 64, True, None), (256, 128, True, None), (128, 256, True, None),
+                                             (128, 64, False, None), (64, 128, True, 1500), (96, 128, False, 2048),
+                                             (64, 256, True, 900), (64, 64, True, 5461), (64, 64, True, 5462)])
+def test_conv1_child_plan_matches_parent_plan(cin, cchild, ln, n):
     """conv1 of the C2S block through the child plan (only active children
     computed) stores exactly what the parent-plan conv1 (all eight children,
     inactive ones dropped) stores -- the same sum in the same order per value,
     whether a tile stages its halo in LDS or, overflowed, gathers from global
     memory -- with 128-channel tiles, with the per-child LayerNorm in the
     tile (128 channels) or
-    through the f32 staging (256).  Children of 64 channels take 64-channel
+    through the f32 staging (256).  The same on few parents, where both plans
+    take the row-block tile (2,048 blocks of 16 rows x 64 channels of all
+    children).  Children of 64 channels take 64-channel
     tiles in the child plan, whose two waves per row half split the stages
-    (another order of the same sum): held to the bf16 bar."""
+    (another order of the same sum), or the row blocks (up to 5,461 parents):
+    held to the bf16 bar."""
     rng = np.random.default_rng(cin + cchild + ln)
-    parents = _c2s_parents()
+    parents = _c2s_parents(n)
     P = len(parents)
     mask = rng.random((P, 8)) < 0.5
     cfg = F.SparseSubmConvConfig(cin, 8 * cchild)
