@@ -229,7 +229,9 @@ static int conv_forward_impl(const sc_conv_config *cfg, int act_dtype, const voi
     // tile's lanes read their residual before they store.
     bool row_fuse = mfma && ln_in_tile(cfg, act_dtype, c2s);
     const int64_t out_bytes = n_q * cfg->out_channels * (int64_t)dtype_size(out_dtype);
-    a.in_place = ranges_overlap(d_input, in_bytes, d_out, out_bytes) ? 1 : 0;
+    // (a child scatter's output has rows and a size of its own, and several
+    // workgroups write a parent's children anyway)
+    a.in_place = !c2s.scatter && ranges_overlap(d_input, in_bytes, d_out, out_bytes) ? 1 : 0;
     if (row_fuse && act_f32 && out_dtype == SC_DTYPE_F32 && !c2s.skip && !a.in_place &&
         !ranges_overlap(d_residual, out_bytes, d_out, out_bytes) &&
         f32_tile(n_q, a.cout_g, groups) < f32_row_tile(a.cout_g)) {

@@ -8,10 +8,13 @@ Against the float64 product of the same rounded operands: bf16 / f16 outputs to
 half an ulp (2^-9, 2^-12 of the value; the bounds below leave a factor of two)
 plus the f32 sum's error; f32 outputs to 2e-5 (a sum of Cin <= 544 products in
 f32, whose error is near sqrt(Cin) 2^-24, about 2e-6)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
+from bevy_synth_amd import _capi
 from bevy_synth_amd import decoder as D
 from bevy_synth_amd import flex_gmm as F
 from tests.test_gpu_plan import dev
@@ -68,3 +71,31 @@ def test_dense_tile_child_lists(n, cin, cout, dtype):
     full = (x.double() @ w.double().T + layer.bias.double()).reshape(n * 8, cout)
     assert_close(got.double().cpu().numpy(), full[torch.from_numpy(np.flatnonzero(on)).cuda()].cpu().numpy(), TOL[dtype])
     assert torch.equal(got, every)
+
+
+@pytest.mark.parametrize("n,cout", [(1000, 128)])  # row blocks
+def test_child_list_of_another_size(n, cout):
+    """Through the C ABI, a linear child plan built for fewer parents: nothing
+    is written, and the plan's check reports it."""
+    on = np.random.default_rng(n).random((n, 8)) < 0.5
+
+    def lists(rows):
+        _, _, child_rows = F.subdivision_build_indexed(dev(shell(n)[:rows]), mask=dev(on[:rows].astype(np.uint8)))
+        return child_rows, F.build_linear_child_plan(child_rows, int(on[:rows].sum())).buf
+    child_rows, own = lists(n)
+    other = torch.zeros_like(own)
+    short = lists(n - 300)[1]
+    other[:len(short)] = short
+    x, w = randn((n, 256), 5).bfloat16(), randn((8 * cout, 256), 6, 1 / 16).bfloat16()
+    out = torch.full((int(on.sum()), cout), 7.0, dtype=torch.bfloat16, device="cuda")
+    epi = _capi.ScConvEpilogue()
+    epi.child_rows, epi.n_child_rows = ctypes.c_void_p(child_rows.data_ptr()), len(out)
+    lib, stream = _capi.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def call(plan):
+        p = [ctypes.c_void_p(t.data_ptr()) for t in (x, w, out, plan)]
+        assert lib.sc_linear_forward_child_planned(1, p[0], n, 256, 8 * cout, 1, p[1], None, None, ctypes.byref(epi),
+                                                   1, p[2], p[3], stream) == 0
+        return lib.sc_conv_plan_check(p[3], stream)
+    assert call(other) == 2 and (out == 7.0).all()
+    assert call(own) == 0 and not (out == 7.0).all()
