@@ -1499,8 +1499,12 @@ __global__ __launch_bounds__(DenseShape<kQ>::kThreads, DenseShape<kQ>::kBlocksPe
     if constexpr (kListed) {
         // the plan's list tiles in use, each with child_ch / kCols column
         // tiles of its child, dealt to the XCDs as one range; the plan must
-        // be the one built for these parents
-        if (!plan_matches(args.plan_hdr, args) || args.plan_hdr->status != 0u) return;
+        // be the one built for these parents (its status records it if not)
+        if (!plan_matches(args.plan_hdr, args)) {
+            flag_plan_status(args.plan_hdr, kPlanStatusMapMismatch);
+            return;
+        }
+        if (args.plan_hdr->status != 0u) return;
         const int n_ct = args.child_ch / S::kCols;
         const int n_real = args.plan_hdr->n_unique * n_ct;
         if ((int)blockIdx.x >= n_real) return;

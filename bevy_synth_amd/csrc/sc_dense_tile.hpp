@@ -80,7 +80,11 @@ __global__ __launch_bounds__(512, 1) void dense_tile_kernel(ConvArgs args)
     int row_tiles, first, n_mine = 0;
     if constexpr (kListed) {
         const PlanHeader *h = args.plan_hdr;
-        row_tiles = plan_matches(h, args) && h->status == 0u ? h->n_unique : 0;
+        if (!plan_matches(h, args)) {
+            flag_plan_status(h, kPlanStatusMapMismatch);
+            return;
+        }
+        row_tiles = __builtin_amdgcn_readfirstlane(h->status == 0u ? h->n_unique : 0);
         if (row_tiles == 0) return;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {

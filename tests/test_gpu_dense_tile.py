@@ -73,7 +73,7 @@ def test_dense_tile_child_lists(n, cin, cout, dtype):
     assert torch.equal(got, every)
 
 
-@pytest.mark.parametrize("n,cout", [(1000, 128)])  # row blocks
+@pytest.mark.parametrize("n,cout", [(1000, 128), (8000, 128), (30000, 256)])  # row blocks, dense_gemm, dense_tile
 def test_child_list_of_another_size(n, cout):
     """Through the C ABI, a linear child plan built for fewer parents: nothing
     is written, and the plan's check reports it."""
