@@ -1371,17 +1371,31 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
     }
 #pragma unroll
     for (int ih = 0; ih < kI; ih += kRG) {
-        typename Out8<TO>::V rv[kRG][2];
+        typename Out4<TO>::V rv[kRG][2][2];
         if (res && vec8) {
 #pragma unroll
             for (int ii = 0; ii < kRG; ++ii)
 #pragma unroll
                 for (int jp = 0; jp < 2; ++jp) {
                     const int oc = oc0 + 32 * jp + 8 * q4;
-                    if (qrow[ih + ii] >= 0 && oc < args.cout_g)
-                        rv[ii][jp] = *reinterpret_cast<const typename Out8<TO>::V *>(
+                    if (qrow[ih + ii] >= 0 && oc < args.cout_g) {
+                        const auto r8 = *reinterpret_cast<const typename Out8<TO>::V *>(
                             res + (int64_t)qrow[ih + ii] * args.cout + out_col0 + oc);
+                        __builtin_memcpy(rv[ii][jp], &r8, sizeof(r8));
+                    }
                 }
+        } else if (res && vec_ok) {
+#pragma unroll
+            for (int ii = 0; ii < kRG; ++ii)
+#pragma unroll
+                for (int jp = 0; jp < 2; ++jp)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int oc = oc0 + 32 * jp + 8 * q4 + 4 * h;
+                        if (qrow[ih + ii] >= 0 && oc + 3 < args.cout_g)
+                            rv[ii][jp][h] = *reinterpret_cast<const typename Out4<TO>::V *>(
+                                res + (int64_t)qrow[ih + ii] * args.cout + out_col0 + oc);
+                    }
         }
 #pragma unroll
         for (int ii = 0; ii < kRG; ++ii) {
@@ -1402,7 +1416,8 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
                 if (vec8) {
                     if (res) {
                         float r8[8];
-                        Out8<TO>::unpack(rv[ii][jp], r8);
+                        Out4<TO>::unpack(rv[ii][jp][0], r8);
+                        Out4<TO>::unpack(rv[ii][jp][1], r8 + 4);
 #pragma unroll
                         for (int cc = 0; cc < 8; ++cc) v[cc] += r8[cc];
                     }
@@ -1413,8 +1428,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
                         if (vec_ok && oc + h + 3 < args.cout_g) {
                             if (res) {
                                 float r4[4];
-                                Out4<TO>::unpack(
-                                    *reinterpret_cast<const typename Out4<TO>::V *>(res + rowbase + oc + h), r4);
+                                Out4<TO>::unpack(rv[ii][jp][h / 4], r4);
 #pragma unroll
                                 for (int cc = 0; cc < 4; ++cc) v[h + cc] += r4[cc];
                             }
