@@ -786,9 +786,10 @@ __global__ __launch_bounds__(kThreads, 2) void conv_v2_kernel(ConvArgs args)
 // Tile = 256 rows x 128 output channels, 4 waves, two workgroups per CU;
 // wave w owns rows [128 (w/2), +128) x channels [64 (w%2), +64) as 8 x 4
 // blocks of v_mfma_f32_16x16x32_bf16 (transposed product: lane l holds
-// channels 4*(l/16)+e of row l%16 of each block; before the stores the lanes of
-// a row trade registers, so that two blocks make 8 consecutive channels, one
-// 16-byte store, residual load or child-row lookup where there were two of 8
+// four channels of row l%16 of each block; the weight rows are dealt to the
+// blocks, or after LayerNorm the lanes of a row trade registers, so that two
+// blocks make 8 consecutive channels, one 16-byte store, residual load or
+// child-row lookup where channels 4*(l/16)+e of each block made two of 8
 // bytes: the residual block of 1,040,679 x 128 1,700 -> 1,667 us, an int8
 // decoder stack 16.66 -> 16.40 ms).  Stage = (32-channel chunk c, used offset
 // k), chunk-major.  Per stage a wave reads 8 operand fragments
@@ -850,6 +851,11 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
     // of at most 64 output channels): waves 2 (row halves) x 2 (stage
     // parity) in the loop, 64 rows x 64 channels each in the epilogue.
     static_assert(kNT == 128 || kNT == 64, "output tile of 128 or 64 channels");
+    // The weight rows are dealt to the MFMA blocks so that a lane ends with 8
+    // consecutive channels of a row per block pair; LayerNorm needs its sums in
+    // the packed order and trades registers after it instead (300,000 x 32 ->
+    // 104 without LayerNorm: dealt 112.5 us, traded 116.3).
+    constexpr bool kDealt = !kLN;
     constexpr bool kKS = kNT == 64;             // stages split between the waves of a row half
     constexpr int kIM = 8;                      // 16-row MFMA blocks per wave in the loop
     constexpr int kI = kNT == 128 ? 8 : 4;      // ... and in the epilogue
@@ -1032,8 +1038,13 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
         const __amdgpu_buffer_rsrc_t w_rsrc =
             make_rsrc(static_cast<const char *>(args.wpack) + kPackHeaderBytes,
                       (uint32_t)((int64_t)args.cin / args.cin_g * n_ot) * w_tile_bytes);
-        const uint32_t w_lane = (uint32_t)(g * n_ot + (o0 >> 7)) * w_tile_bytes +
-                                (uint32_t)((o0 & 127) / 16 + 4 * ch) * kFrag + (uint32_t)(lane * kWLane);
+        // Dealt: MFMA row m = 4 a + b of block j takes channel 32 (j / 2) + 8 a + 4
+        // (j % 2) + b: lane l16 reads fragment 2 (j / 2) + l16 / 8 at lane 8 ((l16 /
+        // 4) % 2) + 4 (j % 2) + l16 % 4 (still 64 contiguous bytes per 4 lanes).
+        const uint32_t w_lane =
+            (uint32_t)(g * n_ot + (o0 >> 7)) * w_tile_bytes +
+            (uint32_t)((o0 & 127) / 16 + 4 * ch + (kDealt ? l16 >> 3 : 0)) * kFrag +
+            (uint32_t)((kDealt ? 8 * ((l16 >> 2) & 1) + (l16 & 3) + 16 * q4 : lane) * kWLane);
         const int n_halo_instr = (U + 15) >> 4;
 
         struct Cursor {
@@ -1064,7 +1075,10 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
             const bool live = u.c < nkc;
             const uint32_t wk = w_lane + (uint32_t)((u.k * nkc + u.c) * 8) * kFrag;
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj) f[jj] = bload16(w_rsrc, live ? wk + (uint32_t)jj * kFrag : kOobOffset);
+            for (int jj = 0; jj < 4; ++jj)
+                f[jj] = bload16(w_rsrc, live ? wk + (kDealt ? (uint32_t)(jj >> 1) * 2 * kFrag + (uint32_t)(jj & 1) * 4 * kWLane
+                                                            : (uint32_t)jj * kFrag)
+                                             : kOobOffset);
         };
         // Halo DMA: instruction wave + 4*ii fills halo rows 16*(wave + 4*ii) + lane/4;
         // the lane moves logical piece hslot(j, lane%4) of row j.  Issued as
@@ -1222,8 +1236,9 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
 
     // ---- epilogue: lane l holds channels oc0 + 16 j + 4 q4 + e of tile row
     //      row0 + 16 i + l16 (LayerNorm's sums add in this order, the same
-    //      as the dense kernels'); the lanes l16 + 16 m of the wave (kNT = 64)
-    //      or of the two waves of a row half (kNT = 128) hold the whole row.
+    //      as the dense kernels'), or dealt, oc0 + 32 (j / 2) + 8 q4 + 4 (j %
+    //      2) + e; the lanes l16 + 16 m of the wave (kNT = 64) or of the two
+    //      waves of a row half (kNT = 128) hold the whole row.
     TO *__restrict__ out = static_cast<TO *>(args.out);
     const TO *__restrict__ res = static_cast<const TO *>(args.residual);
     const bool vec_ok = args.vec_out != 0, vec8 = args.vec_out >= 8;
@@ -1232,7 +1247,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
     for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int o = oc0 + j * 16 + 4 * q4 + e;
+            const int o = oc0 + (kDealt ? 32 * (j >> 1) + 8 * q4 + 4 * (j & 1) : 16 * j + 4 * q4) + e;
             const bool ok = o < args.cout_g;
             const float bias = s_bias[o - o0], scale = s_scale[o - o0];
 #pragma unroll
@@ -1314,20 +1329,22 @@ __global__ __launch_bounds__(kThreads, 2) void conv_halo_kernel(ConvArgs args, P
             }
     }
     // The stores want 8 consecutive channels a lane (16 bytes, the 4 lanes of
-    // a row 64): lane q4 = 2 q1 + q0 trades registers with its row's other
-    // lanes until block pair jp holds channels oc0 + 32 jp + 8 q4 + [0, 8).
-    // 16 instructions per row block, once a tile; every lane takes part.
+    // a row 64).  Not dealt that way, lane q4 = 2 q1 + q0 trades registers with its
+    // row's other lanes until block pair jp holds channels oc0 + 32 jp + 8 q4 +
+    // [0, 8): 16 instructions per row block, once a tile; every lane takes part.
+    if constexpr (!kDealt) {
 #pragma unroll
-    for (int i = 0; i < kI; ++i)
+        for (int i = 0; i < kI; ++i)
 #pragma unroll
-        for (int jp = 0; jp < 2; ++jp)
+            for (int jp = 0; jp < 2; ++jp)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float a = acc[i][2 * jp][e], b = acc[i][2 * jp + 1][e];
-                pair_to_row8(a, b);
-                acc[i][2 * jp][e] = a;
-                acc[i][2 * jp + 1][e] = b;
-            }
+                for (int e = 0; e < 4; ++e) {
+                    float a = acc[i][2 * jp][e], b = acc[i][2 * jp + 1][e];
+                    pair_to_row8(a, b);
+                    acc[i][2 * jp][e] = a;
+                    acc[i][2 * jp + 1][e] = b;
+                }
+    }
     // Stores: the residual of kRG row blocks (4 for bf16, 2 for f32 outputs)
     // is fetched before any of them is written, so its latency overlaps
     // instead of serialising per block.
