@@ -173,6 +173,7 @@ __global__ void nm_header_init_kernel(NbrHeader *h)
     h->status = 0;
     h->unsorted = 0;
     h->mode = 0;
+    h->one_launch = 0;
 }
 
 // Rank bitmap lookup: word w of the bitmap holds the occupancy bits of cells
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(256) void nm_plan_init_kernel(const int32_t *__rest
         const Plan p = make_plan(&s_h, lim);
         s_h.plan = p;
         s_h.mode = p.mode;
-        s_h.pad0 = 0;
+        s_h.one_launch = 0;
     }
     __syncthreads();
     const Plan p = s_h.plan;
@@ -1053,7 +1054,7 @@ __global__ __launch_bounds__(kSmallThreads) void nm_small_kernel(const int4 *__r
             const Plan p = make_plan(&s_h, lim);
             s_h.plan = p;
             s_h.mode = p.mode;
-            s_h.pad0 = 0;
+            s_h.one_launch = 1;
             if (p.mode == 4 && s_dup) s_h.status |= kStatusDupCell;
         }
         __syncthreads();

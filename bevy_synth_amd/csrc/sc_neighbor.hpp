@@ -41,7 +41,7 @@ struct alignas(16) NbrHeader {
     uint32_t status;
     uint32_t unsorted;  // bit L set unless the rows are strictly increasing in the L-level key
     int32_t mode;       // the table mode chosen (Plan::mode), a diagnostic for callers
-    uint32_t pad0;
+    uint32_t one_launch;  // 1: nm_small_kernel's own LDS table was used, not the one `mode` names; a diagnostic
     Plan plan;          // derived once from the fields above, read by every later kernel
     uint8_t pad[kHeaderBytes - 48 - sizeof(Plan)];
 };

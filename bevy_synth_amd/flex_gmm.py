@@ -156,9 +156,17 @@ NEIGHBOR_TABLE_MODES = {1: "hash32", 2: "hash64", 3: "hash_coords", 4: "dense_gr
 
 def neighbor_map_table_mode(workspace: torch.Tensor) -> str:
     """The table the last build into ``workspace`` chose on the device (the
-    int32 at byte 40 of the workspace header); syncs the current stream."""
+    int32 at byte 40 of the workspace header); syncs the current stream.  A
+    small set's build (``neighbor_map_one_launch``) does not write that table."""
     mode = int(workspace[40:44].view(torch.int32).item())
     return NEIGHBOR_TABLE_MODES.get(mode, "none")
+
+
+def neighbor_map_one_launch(workspace: torch.Tensor) -> bool:
+    """Whether the last build into ``workspace`` was the single launch of small
+    sets (at most 4,096 rows and 32 offsets), which looks rows up in a table of
+    its own; syncs the current stream."""
+    return int(workspace[44:48].view(torch.int32).item()) == 1
 
 
 def neighbor_map_rank_levels(workspace: torch.Tensor) -> int:

@@ -118,7 +118,10 @@ int sc_neighbor_map_workspace_size(int64_t n_rows, size_t *bytes);
  * The table is chosen on the device from the coords' bbox and order; the
  * int32 at byte 40 of d_workspace records it after the build (a diagnostic):
  * 1/2 hash table with 32/64-bit keys, 3 hash table over the coords, 4 dense
- * bbox grid, 5 rank bitmap (rows strictly increasing in (b, x, y, z)).
+ * bbox grid, 5 rank bitmap (rows strictly increasing in (b, x, y, z)).  Sets of
+ * at most 4,096 rows and 32 offsets are built in one launch with a hash table
+ * that is never written to d_workspace: the int32 at byte 44 is then 1 (else
+ * 0), and byte 40 tells what a larger set of that bbox and order would take.
  */
 int sc_neighbor_map_build(const sc_conv_config *cfg, const int32_t *d_coords, int64_t n_rows,
                           int64_t query_rows, int32_t *d_map, void *d_workspace,

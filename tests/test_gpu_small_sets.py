@@ -77,7 +77,9 @@ def test_small_order_and_map(oracle, kind, n):
     n = len(coords)
     cfg = F.SparseSubmConvConfig(32, 32)
     cd = dev(coords)
-    nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, cd)
+    ws = F.NeighborMapWorkspace()
+    nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, cd, workspace=ws)
+    assert F.neighbor_map_one_launch(ws.get(n)) == (n <= LIMIT)
     assert np.array_equal(nbr.cpu().numpy(), oracle.build_neighbor_rows_scan(ocfg(oracle, cfg), coords))
     h = check_plan(F.build_conv_plan(cfg, cd, nbr), nbr.cpu().numpy(), n)
     assert h["grid_mode"] == mode
