@@ -700,8 +700,9 @@ template <typename Tin>
 void launch_linear_skinny(const Tin *x, int64_t rows, int cin, const float *w, const float *b, int cout, float *out,
                           hipStream_t s)
 {
-    // whole 16-byte pieces, and a 64-row block's bytes in 32 bits
-    if (cin % Vec16<Tin>::N == 0 && (int64_t)cin * (int64_t)sizeof(Tin) <= 1 << 20) {
+    // whole 16-byte pieces, a 64-row block's bytes in 32 bits, and a thread per
+    // row within a launch's 2^32
+    if (cin % Vec16<Tin>::N == 0 && (int64_t)cin * (int64_t)sizeof(Tin) <= 1 << 20 && rows <= INT32_MAX) {
         const unsigned g = grid_for(rows, 64 * kSkinnyWaves, INT32_MAX);
         linear_skinny_rows_kernel<Tin><<<g, 64 * kSkinnyWaves, 0, s>>>(x, rows, cin, w, b, cout, out);
         return;

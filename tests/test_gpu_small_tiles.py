@@ -220,6 +220,21 @@ def test_skinny_rows_edges(rows, cin, cout, dtype):
     assert_close(got, x.double().cpu().numpy() @ w.T.astype(np.float64) + b, TOL[torch.float32])
 
 
+def test_skinny_more_rows_than_a_launch_has_threads():
+    rows, cin = 2**32 + 3, 8  # 69 GB in, 17 GB out
+    if torch.cuda.mem_get_info()[0] < 100 << 30:
+        pytest.skip("needs 86 GB of free device memory")
+    x = torch.empty((rows, cin), dtype=torch.float16, device="cuda")
+    w = dev(np.arange(1, cin + 1, dtype=np.float32).reshape(1, cin))
+    at = torch.tensor([0, 2**31, 2**32 - 1, 2**32, rows - 1], device="cuda")
+    for i, r in enumerate(at.tolist()):
+        x[r] = i + 1
+    got = F.linear_skinny(x, w)[at].cpu().numpy().ravel()
+    del x
+    torch.cuda.empty_cache()
+    assert np.array_equal(got, 36.0 * np.arange(1, 6))
+
+
 # Cout a multiple of 8 (16-byte stores), of 4, of neither
 @pytest.mark.parametrize("cout,form", [(1024, "plain"), (640, "residual"), (1028, "residual"), (1030, "residual")])
 def test_halo_tiles_few_rows(oracle, cout, form):
