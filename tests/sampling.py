@@ -30,3 +30,10 @@ def sample_rows(n, rng, k=2000, plan=None, extra=()):
     left = min(max(0, k - len(must)), len(pool))
     rand = rng.choice(pool, size=left, replace=False) if left else np.zeros(0, np.int64)
     return np.unique(np.concatenate([must, rand]))
+
+
+def rows_past_row_blocks(cout_g, groups=1):
+    """Rows of a call just past the size that 16-bit calls take on the
+    row-block tile (2,048 blocks of 16 rows x 64 channels): the 256-row tiles
+    take it, the last of them with few rows."""
+    return 16 * (2048 // (-(-cout_g // 64) * groups)) + 21

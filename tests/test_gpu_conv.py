@@ -2,13 +2,16 @@
 
 f32: within 1e-4 of the oracle's flex path and of its fp64 definition.
 bf16 (bf16 operands, f32 accumulate): within 1e-2 of the fp64 definition on
-the same bf16-rounded operands.  Metric: max |a-b| / max(|b|, rms(b))."""
+the same bf16-rounded operands.  Metric: max |a-b| / max(|b|, rms(b)).
+16-bit convs without a plan: the row-block tile (``few`` rows) and the 256-row
+tile just past its limit."""
 import numpy as np
 import pytest
 import torch
 
 from bevy_synth_amd import flex_gmm as F
 from bevy_synth_amd import synth
+from tests.sampling import rows_past_row_blocks, sample_rows
 from tests.tolerance import TOL_BF16, TOL_F32, assert_close
 
 pytestmark = pytest.mark.gpu
@@ -26,6 +29,10 @@ def ocfg(oracle, cfg):
     return oracle.OracleConfig(cfg.in_channels, cfg.out_channels, cfg.kernel_d, cfg.kernel_h,
                                cfg.kernel_w, groups=cfg.groups, axis_order=cfg.axis_order,
                                axis_sign=cfg.axis_sign)
+
+
+def first_rows(n):
+    return np.ascontiguousarray(synth.config2_coords()[:n])
 
 
 def line_coords(n):
@@ -103,8 +110,9 @@ def test_config1_f32_mfma(oracle):
 @pytest.mark.parametrize("cin,cout,groups", [(32, 32, 1), (64, 96, 1), (128, 128, 1),
                                              (256, 64, 1), (64, 64, 2), (96, 200, 1)])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
-def test_bf16_mfma_shapes(oracle, cin, cout, groups, out_dtype):
-    coords = synth.config1_coords()[:6000]
+@pytest.mark.parametrize("few", [True, False])
+def test_bf16_mfma_shapes(oracle, cin, cout, groups, out_dtype, few):
+    coords = first_rows(6000 if few else rows_past_row_blocks(cout // groups, groups))
     rng = np.random.default_rng(cin * 7 + cout + groups)
     n = len(coords)
     x = synth.bf16_to_f32(synth.bf16_bits(synth.normal_f32(rng, (n, cin))))
@@ -114,15 +122,17 @@ def test_bf16_mfma_shapes(oracle, cin, cout, groups, out_dtype):
     cfg = F.SparseSubmConvConfig(cin, cout, groups=groups)
     nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, dev(coords))
     out = F.sparse_subm_conv_forward(cfg, bf16_dev(x), nbr, bf16_dev(w), dev(b), out_dtype=out_dtype)
-    got = out.float().cpu().numpy()
-    exp = oracle.conv_ref_f64(ocfg(oracle, cfg), w, b, x, nbr.cpu().numpy())
+    rows = np.arange(n) if few else sample_rows(n, rng, 2000)
+    got = out.float().cpu().numpy()[rows]
+    exp = oracle.conv_ref_f64(ocfg(oracle, cfg), w, b, x, nbr.cpu().numpy()[rows])
     assert_close(got, exp, TOL_BF16 if out_dtype == torch.bfloat16 else 2e-5, "bf16 conv")
 
 
-def test_int8_weights_w8a16(oracle):
-    coords = synth.config1_coords()[:5000]
+@pytest.mark.parametrize("cin,cout,n", [(128, 64, 5000), (128, 64, None), (64, 200, None)])
+def test_int8_weights_w8a16(oracle, cin, cout, n):
+    coords = first_rows(n or rows_past_row_blocks(cout))
     rng = np.random.default_rng(5)
-    n, cin, cout = len(coords), 128, 64
+    n = len(coords)
     x = synth.bf16_to_f32(synth.bf16_bits(synth.normal_f32(rng, (n, cin))))
     q, scale = synth.int8_weight(rng, cout, 27, cin)
     b = synth.normal_f32(rng, cout, 0.1)
@@ -130,9 +140,30 @@ def test_int8_weights_w8a16(oracle):
     nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, dev(coords))
     out = F.sparse_subm_conv_forward(cfg, bf16_dev(x), nbr, dev(q), dev(b), w_scale=dev(scale),
                                      out_dtype=torch.float32)
-    exp = oracle.conv_ref_f64(ocfg(oracle, cfg), q.astype(np.float32), b, x, nbr.cpu().numpy(),
+    rows = sample_rows(n, rng, 5000)
+    exp = oracle.conv_ref_f64(ocfg(oracle, cfg), q.astype(np.float32), b, x, nbr.cpu().numpy()[rows],
                               w_scale=scale)
-    assert_close(out.cpu().numpy(), exp, 2e-5, "int8 conv")
+    assert_close(out.cpu().numpy()[rows], exp, 2e-5, "int8 conv")
+
+
+@pytest.mark.parametrize("cout", [64, 96, 128])
+def test_unplanned_layer_norm_in_the_tile(oracle, cout):
+    """conv -> LN -> SiLU -> + residual on the 256-row tile without a plan."""
+    coords = first_rows(rows_past_row_blocks(cout))
+    rng = np.random.default_rng(cout)
+    n, cin = len(coords), 64
+    x = synth.bf16_to_f32(synth.bf16_bits(synth.normal_f32(rng, (n, cin))))
+    w = synth.bf16_to_f32(synth.bf16_bits(synth.conv_weight(rng, cout, 27, cin, 1.0 / np.sqrt(27 * cin))))
+    b, lw, lb = (synth.normal_f32(rng, cout) for _ in range(3))
+    res = synth.normal_f32(rng, (n, cout))
+    cfg = F.SparseSubmConvConfig(cin, cout)
+    nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, dev(coords))
+    out = F.sparse_subm_conv_forward(cfg, bf16_dev(x), nbr, bf16_dev(w), dev(b), residual=dev(res), layer_norm=True,
+                                     ln_weight=dev(lw), ln_bias=dev(lb), silu=True, out_dtype=torch.float32)
+    rows = sample_rows(n, rng, 2000)
+    conv = oracle.conv_ref_f64(ocfg(oracle, cfg), w, b, x, nbr.cpu().numpy()[rows]).astype(np.float32)
+    exp = oracle.silu(oracle.layer_norm(conv, lw, lb, 1e-6)) + res[rows]
+    assert_close(out.cpu().numpy()[rows], exp, 1e-4, "LayerNorm, 256-row tile")
 
 
 def test_k1_is_dense_gemm():
@@ -150,20 +181,22 @@ def test_k1_is_dense_gemm():
     assert_close(out.cpu().numpy(), ref.numpy(), 2e-5, "k1 gemm")
 
 
-def test_residual_and_query_subset(oracle):
-    coords = synth.config1_coords()
+@pytest.mark.parametrize("q", [5000, 32789])
+def test_residual_and_query_subset(oracle, q):
+    coords = synth.config1_coords() if q == 5000 else first_rows(40000)
     rng = np.random.default_rng(4)
     n, c = len(coords), 64
     x = synth.bf16_to_f32(synth.bf16_bits(synth.normal_f32(rng, (n, c))))
     w = synth.bf16_to_f32(synth.bf16_bits(synth.conv_weight(rng, c, 27, c, 0.03)))
     b = synth.normal_f32(rng, c, 0.1)
-    res = synth.normal_f32(rng, (5000, c))
+    res = synth.normal_f32(rng, (q, c))
     cfg = F.SparseSubmConvConfig(c, c)
-    nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, dev(coords), query_rows=5000)
+    nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, dev(coords), query_rows=q)
     out = F.sparse_subm_conv_forward(cfg, bf16_dev(x), nbr, bf16_dev(w), dev(b),
                                      residual=dev(res), out_dtype=torch.float32)
-    exp = oracle.conv_ref_f64(ocfg(oracle, cfg), w, b, x, nbr.cpu().numpy()) + res
-    assert_close(out.cpu().numpy(), exp, 2e-5, "residual")
+    rows = sample_rows(q, rng, 5000)
+    exp = oracle.conv_ref_f64(ocfg(oracle, cfg), w, b, x, nbr.cpu().numpy()[rows]) + res[rows]
+    assert_close(out.cpu().numpy()[rows], exp, 2e-5, "residual")
 
 
 def test_isolated_rows_get_bias():

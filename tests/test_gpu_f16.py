@@ -14,7 +14,7 @@ import torch
 
 from bevy_synth_amd import flex_gmm as F
 from bevy_synth_amd import synth
-from tests.sampling import sample_rows
+from tests.sampling import rows_past_row_blocks, sample_rows
 from tests.tolerance import TOL_BF16, assert_close, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -69,12 +69,16 @@ def test_config1_conv_f16(oracle, planned, out_dtype):
     assert e <= (1e-3 if out_dtype == torch.float16 else 1e-4), e
 
 
-@pytest.mark.parametrize("kernel,n", [((3, 3, 1), 14648), ((1, 1, 1), 14648), ((3, 3, 3), 257)])
+@pytest.mark.parametrize("kernel,n", [((3, 3, 1), 14648), ((1, 1, 1), 14648), ((3, 3, 3), 257),
+                                      ((3, 3, 1), None), ((1, 1, 1), None), ((3, 3, 3), None)])
 @pytest.mark.parametrize("cout", [64, 128])
 def test_f16_planned_few_offsets_and_rows(oracle, kernel, n, cout):
-    """The planned f16 tile on plans over 9 and 1 offsets, and on 257 rows
-    (a full tile then a one-row tile), at both tile widths."""
-    coords = np.ascontiguousarray(synth.config1_coords()[:n])
+    """The planned f16 conv on plans over 27, 9 and 1 offsets: the halo-staged
+    tiles of both widths (n None: just past the row blocks' limit), and the
+    row-block tile up to 257 rows (a full plan tile then a one-row one)."""
+    few = n is not None
+    n = n or rows_past_row_blocks(cout)
+    coords = np.ascontiguousarray(synth.config2_coords()[:n])
     rng = np.random.default_rng(n + cout + sum(kernel))
     cin = 64
     K = kernel[0] * kernel[1] * kernel[2]
@@ -85,30 +89,33 @@ def test_f16_planned_few_offsets_and_rows(oracle, kernel, n, cout):
     cd = dev(coords)
     nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, cd)
     wd = f16_dev(w)
-    got = F.sparse_subm_conv_forward(cfg, f16_dev(x), nbr, wd, dev(b), out_dtype=torch.float16,
-                                     plan=F.build_conv_plan(cfg, cd, nbr),
+    plan = F.build_conv_plan(cfg, cd, nbr)
+    got = F.sparse_subm_conv_forward(cfg, f16_dev(x), nbr, wd, dev(b), out_dtype=torch.float16, plan=plan,
                                      packed_weight=F.pack_conv_weight(cfg, wd))
-    exp = oracle.conv_gemm_f64(oracle.OracleConfig(cin, cout, *kernel), w, b, x, nbr.cpu().numpy())
-    assert_close(host(got), exp, TOL_BF16, f"f16 planned conv, kernel {kernel}, {n} rows")
+    rows = np.arange(n) if few else sample_rows(n, rng, 3000, plan=plan)
+    exp = oracle.conv_gemm_f64(oracle.OracleConfig(cin, cout, *kernel), w, b, x, nbr.cpu().numpy()[rows])
+    assert_close(host(got)[rows], exp, TOL_BF16, f"f16 planned conv, kernel {kernel}, {n} rows")
 
 
 @pytest.mark.parametrize("cout", [64, 128])
-def test_f16_planned_overflow_tiles(oracle, cout):
-    """The f16 tile with some tiles over the halo budget (cluster centres
-    whose 26 neighbours are all distinct): those tiles gather their operands
-    from global memory in the same launch; every row against the fp64
-    definition, both tile widths."""
-    side = 7
-    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:300]
+@pytest.mark.parametrize("few", [True, False])
+def test_f16_planned_overflow_tiles(oracle, cout, few):
+    """The f16 halo-staged tile with some tiles over the halo budget (cluster
+    centres whose 26 neighbours are all distinct): those tiles gather their
+    operands from global memory in the same launch; against the fp64
+    definition, both tile widths (few: every row, on the row-block tile)."""
+    q = 3300 if few else rows_past_row_blocks(cout)
+    n_c = q // 11
+    side = int(np.ceil(n_c ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n_c]
     centres = 200 + 3 * g
     offs = np.stack(np.meshgrid(*[np.arange(-1, 2)] * 3, indexing="ij"), -1).reshape(-1, 3)
     offs = offs[np.any(offs != 0, axis=1)]
     nb = (centres[:, None, :] + offs[None]).reshape(-1, 3)
-    shell = synth.config1_coords()[:3000]
+    shell = synth.config2_coords()[:q - n_c]
     xyz = np.concatenate([centres, nb])
     cl = np.concatenate([np.zeros((len(xyz), 1), np.int32), xyz.astype(np.int32)], 1)
-    coords = np.ascontiguousarray(np.concatenate([shell, cl[:300], cl[300:]]))
-    q = 3300
+    coords = np.ascontiguousarray(np.concatenate([shell, cl[:n_c], cl[n_c:]]))
     rng = np.random.default_rng(cout + 5)
     cin = 64
     x = _fence(oracle, synth.normal_f32(rng, (len(coords), cin)))
@@ -123,8 +130,9 @@ def test_f16_planned_overflow_tiles(oracle, cout):
     wd = f16_dev(w)
     got = F.sparse_subm_conv_forward(cfg, f16_dev(x), nbr, wd, dev(b), out_dtype=torch.float32,
                                      plan=plan, packed_weight=F.pack_conv_weight(cfg, wd))
-    exp = oracle.conv_gemm_f64(oracle.OracleConfig(cin, cout), w, b, x, nbr.cpu().numpy())
-    assert_close(host(got), exp, 2e-5, f"f16 planned conv with overflow tiles, Cout {cout}")
+    rows = np.arange(q) if few else sample_rows(q, rng, 3000, plan=plan)
+    exp = oracle.conv_gemm_f64(oracle.OracleConfig(cin, cout), w, b, x, nbr.cpu().numpy()[rows])
+    assert_close(host(got)[rows], exp, 2e-5, f"f16 planned conv with overflow tiles, Cout {cout}")
 
 
 def test_config2_conv_f16_planned(oracle):
@@ -188,10 +196,12 @@ def test_config3_residual_block_f16(oracle):
 
 
 @pytest.mark.parametrize("cout", [256, 96])
-def test_f16_wide_and_narrow_layer_norm(oracle, cout):
+@pytest.mark.parametrize("few", [True, False])
+def test_f16_wide_and_narrow_layer_norm(oracle, cout, few):
     """conv -> LN -> SiLU with an f16 output: over 256 channels on the f32
-    staging (row kernel), over 96 in the tile epilogue."""
-    coords = synth.config1_coords()[:6000]
+    staging (row kernel), over 96 in the tile epilogue (few: the row-block
+    tile, else the 256-row tiles without a plan)."""
+    coords = np.ascontiguousarray(synth.config2_coords()[:6000 if few else rows_past_row_blocks(cout)])
     rng = np.random.default_rng(cout)
     cin = 64
     x = _fence(oracle, synth.normal_f32(rng, (len(coords), cin)))
@@ -200,10 +210,11 @@ def test_f16_wide_and_narrow_layer_norm(oracle, cout):
     cfg = F.SparseSubmConvConfig(cin, cout)
     nbr = F.neighbor_rows_tensor_from_coords_tensor(cfg, dev(coords))
     got = F.sparse_subm_conv_forward(cfg, f16_dev(x), nbr, f16_dev(w), dev(b), layer_norm=True, silu=True)
-    conv = oracle.conv_gemm_f64(oracle.OracleConfig(cin, cout), w, b, x, nbr.cpu().numpy()).astype(np.float32)
+    rows = np.arange(len(coords)) if few else sample_rows(len(coords), rng, 3000)
+    conv = oracle.conv_gemm_f64(oracle.OracleConfig(cin, cout), w, b, x, nbr.cpu().numpy()[rows]).astype(np.float32)
     exp = oracle.silu(oracle.layer_norm(conv, None, None, 1e-6))
-    assert_close(host(got), exp, TOL_BF16, f"f16 LN over {cout}")
-    assert rel_err(host(got), exp) <= 2e-3
+    assert_close(host(got)[rows], exp, TOL_BF16, f"f16 LN over {cout}")
+    assert rel_err(host(got)[rows], exp) <= 2e-3
 
 
 def test_f16_child_scatter_ln(oracle):

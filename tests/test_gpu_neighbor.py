@@ -1,6 +1,8 @@
 """GPU parity: the HIP neighbour map is bit-exact against the oracle (device
 semantics: lowest row on duplicated coords), on the reference's own test
-shapes and on the benchmark geometries."""
+shapes and on the benchmark geometries.  Sets of at most 4,096 rows (and 32
+offsets) are built in one launch with a table of its own; the tests of the
+larger build's tables have sets above that too."""
 import numpy as np
 import pytest
 import torch
@@ -100,17 +102,21 @@ def _wide_coords(rng, n, scale_axes):
 
 @pytest.mark.parametrize("scale_axes,lo,hi", [((0,), 2.0 ** 32, 2.0 ** 64),
                                               ((0, 1, 2), 2.0 ** 64, np.inf)])
-def test_wide_coordinates(oracle, scale_axes, lo, hi):
+@pytest.mark.parametrize("n", [4000, 6000])
+def test_wide_coordinates(oracle, scale_axes, lo, hi, n):
     """Bboxes of more than 2^32 cells use 64-bit keys; beyond 2^64 cells the
-    row-only table compares coords directly."""
-    c = _wide_coords(np.random.default_rng(3), 4000, scale_axes)
+    row-only table compares coords directly (4,000 rows: the one-launch
+    build's table, which always does)."""
+    c = _wide_coords(np.random.default_rng(3), n, scale_axes)
     span = [float(c[:, j].max() - c[:, j].min() + 1) for j in range(4)]
     cells = float(np.prod(np.array(span, dtype=np.float64)))
     assert lo < cells < hi
     cfg = F.SparseSubmConvConfig(1, 1)
     exp = oracle.build_neighbor_rows(ocfg(oracle, cfg), c)
     assert (exp >= 0).sum() > len(c)
-    assert np.array_equal(gpu_map(cfg, c), exp)
+    got, mode = _map_and_mode(cfg, c, one_launch=n <= 4096)
+    assert mode == ("hash_coords" if np.isinf(hi) else "hash64")
+    assert np.array_equal(got, exp)
 
 
 def test_sparse_bbox_uses_hash_table(oracle):
@@ -181,13 +187,14 @@ def test_shuffled_rows_relabel_consistently(oracle):
     assert np.array_equal(shuf, relabeled)
 
 
-def _map_and_mode(cfg, coords, query_rows=None):
+def _map_and_mode(cfg, coords, query_rows=None, one_launch=None):
     c = dev(coords.astype(np.int32))
     ws = F.NeighborMapWorkspace(c.device).get(len(coords))
     q = len(coords) if query_rows is None else query_rows
     out = torch.empty((q, F.kernel_rows(cfg)), dtype=torch.int32, device=c.device)
     F.neighbor_map_build_into(cfg, c, out, ws, q)
     F.neighbor_map_check(ws)
+    assert one_launch is None or F.neighbor_map_one_launch(ws) == one_launch
     return out.cpu().numpy(), F.neighbor_map_table_mode(ws)
 
 
@@ -339,12 +346,17 @@ def test_config3_shuffled_takes_dense_grid(oracle):
 
 @pytest.mark.parametrize("kernel", [(3, 3, 3), (3, 3, 1), (1, 1, 1), (2, 2, 2), (5, 5, 5), (1, 3, 5)])
 @pytest.mark.parametrize("seed", [0, 1, 2])
-def test_rank_bitmap_small_dense_bboxes(oracle, kernel, seed):
+@pytest.mark.parametrize("large", [False, True])
+def test_rank_bitmap_small_dense_bboxes(oracle, kernel, seed, large):
     """Sorted unique coords in small bboxes (rows at every face and corner of
     the bbox, 32-cell words crossed by neighbour runs, a partial last word,
-    a batch holding one voxel): the rank bitmap against the oracle."""
+    a batch holding one voxel): the rank bitmap against the oracle, on sets
+    above 4,096 rows (large) and of more than 32 offsets; the one-launch build
+    otherwise."""
     rng = np.random.default_rng(100 + seed)
     ext = rng.integers(1, 12, 3)
+    if large:
+        ext[seed] += 25000 // (int(np.prod(ext)) // int(ext[seed]))
     cells = np.stack(np.meshgrid(*[np.arange(e) for e in ext], indexing="ij"), -1).reshape(-1, 3)
     keep = rng.random(len(cells)) < rng.uniform(0.2, 0.9)
     c = np.zeros((int(keep.sum()) + 1, 4), np.int32)
@@ -352,22 +364,27 @@ def test_rank_bitmap_small_dense_bboxes(oracle, kernel, seed):
     c[-1] = [1, 3, 2, 1]                                       # second batch, one voxel
     c = np.unique(c, axis=0)
     cfg = F.SparseSubmConvConfig(1, 1, *kernel)
-    got, mode = _map_and_mode(cfg, c)
+    got, mode = _map_and_mode(cfg, c, one_launch=not large and kernel != (5, 5, 5))
     assert mode == "rank_bitmap"
     assert np.array_equal(got, oracle.build_neighbor_rows(ocfg(oracle, cfg), c))
 
 
 @pytest.mark.parametrize("kernel", [(3, 3, 3), (3, 3, 1), (1, 1, 1), (2, 2, 2), (1, 3, 5), (5, 5, 5)])
 @pytest.mark.parametrize("seed", [0, 1, 2])
-def test_dense_grid_sweep_shuffled(oracle, kernel, seed):
+@pytest.mark.parametrize("large", [False, True])
+def test_dense_grid_sweep_shuffled(oracle, kernel, seed, large):
     """Unique coords in a random row order take the dense grid, whose query
     sweeps the grid's cells (64 cells of a z line per wave unit) and writes
     each row's map row through LDS: z extents below, at and across 64 cells,
     several batches, every axis order and sign draw, and partial queries on
     both sides of the sweep's half-the-rows threshold, against the oracle.
-    K = 125 exceeds the sweep's 32 entries and takes the per-entry query."""
+    K = 125 exceeds the sweep's 32 entries and takes the per-entry query.  The
+    sweep takes sets above 4,096 rows (large), the one-launch build the others
+    of at most 32 offsets."""
     rng = np.random.default_rng(200 + seed)
     ext = np.array([rng.integers(1, 9), rng.integers(1, 9), [1, 64, 97][seed]])
+    if large:
+        ext[:2] = [[180, 170], [30, 11], [13, 27]][seed]
     cells = np.stack(np.meshgrid(*[np.arange(e) for e in ext], indexing="ij"), -1).reshape(-1, 3)
     parts = []
     for b in range(1 + seed):
@@ -382,8 +399,9 @@ def test_dense_grid_sweep_shuffled(oracle, kernel, seed):
     sign = tuple(int(v) for v in rng.choice([-1, 1], 3))
     cfg = F.SparseSubmConvConfig(1, 1, *kernel, axis_order=order, axis_sign=sign)
     exp = oracle.build_neighbor_rows(ocfg(oracle, cfg), c)
-    got, mode = _map_and_mode(cfg, c)
+    got, mode = _map_and_mode(cfg, c, one_launch=len(c) <= 4096 and kernel != (5, 5, 5))
     assert mode == "dense_grid"
+    assert len(c) > 4096 or not large
     assert np.array_equal(got, exp)
     for q in (len(c) * 3 // 5, len(c) // 3, 1):
         got, mode = _map_and_mode(cfg, c, query_rows=q)
