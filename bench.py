@@ -616,11 +616,11 @@ def main():
     ms_map = events_ms(map_build, args.steps, wu)
     ms_plan = events_ms(plan_build, args.steps, wu)
     ms_ln = events_ms(ln_silu, args.steps, wu)
-    # The same map and plan calls on the first 256 rows (sorted and unique
-    # like the whole set, so the same table and row-order modes), where every
-    # kernel has next to nothing to do: the per-call floor of the launch
-    # chain as a Python caller sees it (the host's per-call cost bounds it
-    # when that exceeds the kernels' time).
+    # The same map and plan calls on the first 256 rows: what a call costs a
+    # Python caller when its kernels have next to nothing to do (the host's
+    # per-call cost bounds it when that exceeds the kernels' time).  A set of at
+    # most 4,096 rows takes one launch for the map and two for the plan, not the
+    # four and eight of the whole set.
     n_t = 256
     cd_t = st.coords_d[:n_t].contiguous()
     nbr_t = torch.empty((n_t, 27), dtype=torch.int32, device=dev)
