@@ -108,22 +108,25 @@ def test_linear_skinny(dtype, cin, cout):
 
 
 def _parents_and_mask(n=6000, frac=0.45, seed=3):
-    coords = synth.config1_coords()[:n]
+    coords = (synth.config1_coords() if n <= 14648 else synth.config2_coords())[:n]
     rng = np.random.default_rng(seed)
     mask = (rng.random((len(coords), 8)) < frac).astype(np.uint8)
     return coords, mask
 
 
-@pytest.mark.parametrize("cchild,ln", [(16, True), (64, True), (128, True), (256, True), (64, False),
-                                       (24, True), (96, False)])
+@pytest.mark.parametrize("cchild,ln,n", [(16, True, 6000), (64, True, 6000), (128, True, 6000), (256, True, 6000),
+                                         (64, False, 6000), (24, True, 6000), (96, False, 6000),
+                                         (16, True, 16500), (24, True, 11000), (12, False, 16500),  # 256-row tiles
+                                         (64, True, 1500), (128, True, 1500), (96, False, 1500)])   # row blocks
 @pytest.mark.parametrize("planned", [False, True])
-def test_conv1_child_scatter(oracle, cchild, ln, planned):
+def test_conv1_child_scatter(oracle, cchild, ln, n, planned):
     """conv1 (Cin -> 8*C) on the parents writes child c of parent p to row
     child_rows[p, c], normalised over its C channels: in the tile epilogue
     (C = 64: one wave half; C = 128: the tile) or on f32 staging (C = 16, 24,
     256); C = 24 and 96 take the epilogue's division form (C not a power of
-    two)."""
-    coords, mask = _parents_and_mask()
+    two).  6,000 parents: the 256-row tiles from C = 64 on, below that the row
+    blocks."""
+    coords, mask = _parents_and_mask(n)
     rng = np.random.default_rng(cchild)
     cin, cout = 64, 8 * cchild
     x = rbf(synth.normal_f32(rng, (len(coords), cin)))
@@ -141,22 +144,25 @@ def test_conv1_child_scatter(oracle, cchild, ln, planned):
     got = F.sparse_subm_conv_forward(cfg, bf16_dev(x), nbr, wd, dev(b), layer_norm=ln, silu=ln,
                                      child_rows=rows, n_child_rows=A, **kw)
     assert tuple(got.shape) == (A, cchild)
-    conv = oracle.conv_gemm_f64(oracle.OracleConfig(cin, cout), w, b, x, nbr.cpu().numpy())
     lin = li.cpu().numpy()
-    sl = conv.reshape(len(coords), 8, cchild)[lin // 8, lin % 8].astype(np.float32)
+    at = np.flatnonzero(np.isin(lin // 8, np.r_[:3000, len(coords) - 3000:len(coords)]) if n > 6000 else lin >= 0)
+    par = np.unique(lin[at] // 8)
+    conv = oracle.conv_gemm_f64(oracle.OracleConfig(cin, cout), w, b, x, nbr.cpu().numpy()[par])
+    sl = conv.reshape(len(par), 8, cchild)[np.searchsorted(par, lin[at] // 8), lin[at] % 8].astype(np.float32)
     exp = oracle.silu(oracle.layer_norm(sl, None, None, 1e-6)) if ln else sl
-    assert_close(host(got), exp, TOL_BF16, f"child scatter C={cchild}")
+    assert_close(host(got)[at], exp, TOL_BF16, f"child scatter C={cchild}")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("cin,cchild,ln", [(512, 256, False), (64, 64, True), (96, 128, True), (64, 256, True),
-                                           (32, 24, False)])
+                                           (32, 24, False), (64, 24, False)])
 def test_linear_child_scatter(oracle, dtype, cin, cchild, ln):
     """The 2x2x2 transposed upsample's linear form (sc_linear_forward with
     child_rows): row p's slice c of x W^T + b lands in row child_rows[p, c],
     normalised over its C channels with a [C] affine when asked (C = 64 and
-    128 in the dense tile's epilogue for bf16 / f16, else on f32 staging)."""
-    coords, mask = _parents_and_mask(n=5000, frac=0.45, seed=cin + cchild)
+    128 in the dense tile's epilogue for bf16 / f16, else on f32 staging).  C = 24
+    takes the division form, on the row blocks (Cin 32) and the dense tile."""
+    coords, mask = _parents_and_mask(n=11000 if (cin, cchild) == (64, 24) else 5000, frac=0.45, seed=cin + cchild)
     rng = np.random.default_rng(cin * cchild)
     cout = 8 * cchild
     rnd = {torch.bfloat16: oracle.bf16_round, torch.float16: oracle.f16_round,
@@ -180,13 +186,16 @@ def test_linear_child_scatter(oracle, dtype, cin, cchild, ln):
     assert_close(host(got), exp, tol, f"linear child scatter {cin}->8x{cchild}")
 
 
-@pytest.mark.parametrize("cp,cout", [(512, 256), (128, 64), (64, 128), (256, 32), (128, 32), (256, 96)])
-def test_conv2_parent_skip(oracle, cp, cout):
+@pytest.mark.parametrize("cp,cout", [(512, 256), (128, 64), (64, 128), (256, 32), (128, 32), (256, 96), (64, 160),
+                                     (64, 96)])
+@pytest.mark.parametrize("n", [500, 8400])
+def test_conv2_parent_skip(oracle, cp, cout, n):
     """conv2 on the children + the channel-repeated parent skip in its epilogue
     (S = Cp/8 parent channels per child, each repeated R = Cout/S times):
     R = 4, 4, 16 (one parent load per 4 channels), R = 1, 2 (a load per
-    channel) and R = 3 (the division form)."""
-    coords, mask = _parents_and_mask(3000, 0.5, seed=cp)
+    channel) and R = 3, 20, 12 (the division form).  About 4 n children: the row
+    blocks, and past their limit the halo-staged tiles."""
+    coords, mask = _parents_and_mask(n, 0.5, seed=cp)
     rng = np.random.default_rng(cp + cout)
     cd = dev(coords)
     cc, li, _ = F.subdivision_build(cd, mask=dev(mask), with_pairs=False)
@@ -203,10 +212,11 @@ def test_conv2_parent_skip(oracle, cp, cout):
                                      skip_index=li, plan=plan, packed_weight=F.pack_conv_weight(cfg, wd))
     lin = li.cpu().numpy()
     S = cp // 8
-    skip = parent.reshape(len(coords), 8, S)[lin // 8, lin % 8]
-    exp = oracle.conv_gemm_f64(oracle.OracleConfig(cout, cout), w, b, h, nbr.cpu().numpy()) + \
+    rows = sample_rows(A, rng, 6000, plan=plan)
+    skip = parent.reshape(len(coords), 8, S)[lin[rows] // 8, lin[rows] % 8]
+    exp = oracle.conv_gemm_f64(oracle.OracleConfig(cout, cout), w, b, h, nbr.cpu().numpy()[rows]) + \
         oracle.repeat_interleave(skip, cout // S)
-    assert_close(host(got), exp, TOL_BF16, "conv + parent skip")
+    assert_close(host(got)[rows], exp, TOL_BF16, "conv + parent skip")
 
 
 def test_linear_child_scatter_no_active_child():

@@ -259,7 +259,8 @@ def test_transposed_upsample_matches_oracle(oracle):
 @pytest.mark.parametrize("planned", [False, True])
 def test_fused_conv_ln_silu_residual(oracle, cin, cout, groups, dtype, affine, planned):
     """conv -> LN -> SiLU -> + residual through sc_subm_conv_forward_fused /
-    _planned: in the kernel epilogue (Cout <= 128, MFMA tile), and for wider
+    _planned: in the kernel epilogue (Cout <= 128, MFMA tile; the 5,000 f32
+    rows through the output, and 16 bits on the row blocks), and for wider
     rows (Cout 256 / 512, groups 2) on the f32 conv output staged in the
     epilogue workspace (bf16 output) or in the output itself (f32), then one
     row kernel; Cin = 6 takes the scalar conv.  Every case is held to the
